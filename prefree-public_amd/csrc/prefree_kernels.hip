@@ -474,10 +474,52 @@ struct RowsReduceLds : ReduceLds<T, WCAP, BCAP> {
     T bs[BCAP];
 };
 
+// A row of at most kThreadMax products, in nnz order, its LDS reads four at a
+// time: one latency per four products instead of one per product.  Products
+// past the row add +0, which leaves the sum as it is (it starts at +0, so it
+// is never -0).  Reads up to kSumPad products past the row: the product
+// buffers hold that many more.
+constexpr int kSumPad = 3;
+
+template <typename P>
+__device__ __forceinline__ P short_row_sum(const P *s, int len)
+{
+    P acc = P(0);
+    for (int q = 0; q < len; q += 4) {
+        const P p0 = s[q], p1 = s[q + 1], p2 = s[q + 2], p3 = s[q + 3];
+        acc += p0;
+        acc += q + 1 < len ? p1 : P(0);
+        acc += q + 2 < len ? p2 : P(0);
+        acc += q + 3 < len ? p3 : P(0);
+    }
+    return acc;
+}
+
+// A listed row's products s[a, b) by a group of kRowLanes lanes, four rows per
+// wave at once; the value, on every lane of the group, is the one wave_sum over
+// lane-strided products gives, bit for bit: lane q's slots q, q + 16, q + 32 and
+// q + 48 stand for those lanes of a wave.  Whole wave active; a == b for a group
+// without a row.
+constexpr int kRowLanes = 16;
+
+template <typename P>
+__device__ __forceinline__ P group_row_sum(const P *s, int a, int b, int q)
+{
+    P r[4] = {P(0), P(0), P(0), P(0)};
+    for (int e = a + q; e < b; e += kWave) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (e + j * kRowLanes < b) r[j] += s[e + j * kRowLanes];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = group_sum<kRowLanes>(r[j]);
+    return (r[0] + r[1]) + (r[2] + r[3]);
+}
+
 // Row sums of a tile whose products sit in s_prod (index = nnz - base).
 // bounds(i, ra, rb) gives row_ptr[r], row_ptr[r+1] of local row i; put(i, s)
 // stores the sum.  Rows of <= kThreadMax products: one lane each, summed in
-// nnz order; <= kWaveMax: one wave each (DPP sum); longer: the workgroup.
+// nnz order; <= kWaveMax: sixteen lanes each (DPP sums); longer: the workgroup.
 // Whole workgroup; L.nw / L.nb must be 0 on entry and are 0 again on exit.
 template <typename T, int WCAP, int BCAP, typename Bounds, typename Put>
 __device__ __forceinline__ void reduce_tile(const T *s_prod, ReduceLds<T, WCAP, BCAP> &L, int base, int A, int B,
@@ -494,10 +536,7 @@ __device__ __forceinline__ void reduce_tile(const T *s_prod, ReduceLds<T, WCAP, 
         const int a0 = ra - base;
         const int len = rb - ra;
         if (len <= kThreadMax) {
-            T s = T(0);
-            for (int q = 0; q < len; ++q)
-                s += s_prod[a0 + q];
-            put(i, s);
+            put(i, short_row_sum(s_prod + a0, len));
         } else if (len <= kWaveMax) {
             const int j = atomicAdd(&L.nw, 1);
             if (j < WCAP) { L.wl[j] = i; L.wa[j] = a0; L.wb[j] = a0 + len; }
@@ -508,13 +547,12 @@ __device__ __forceinline__ void reduce_tile(const T *s_prod, ReduceLds<T, WCAP, 
     }
     lds_sync();
     const int nw = min(L.nw, WCAP);
-    for (int j = wave; j < nw; j += kWaves) {
-        T s = T(0);
-        for (int q = L.wa[j] + lane; q < L.wb[j]; q += kWave)
-            s += s_prod[q];
-        s = wave_sum(s);
-        if (lane == 0)
-            put(L.wl[j], s);
+    for (int j0 = wave * (kWave / kRowLanes); j0 < nw; j0 += kWaves * (kWave / kRowLanes)) {
+        const int j = j0 + lane / kRowLanes;
+        const int jc = min(j, nw - 1);
+        const T s = group_row_sum(s_prod, L.wa[jc], j < nw ? L.wb[jc] : 0, lane & (kRowLanes - 1));
+        if (j < nw && (lane & (kRowLanes - 1)) == 0)
+            put(L.wl[jc], s);
     }
     const int nb = min(L.nb, BCAP);
     for (int j = 0; j < nb; ++j) {
@@ -547,7 +585,7 @@ template <typename T, bool MERGE, int K, int LMAX>
 __global__ __launch_bounds__(kBS) void k_tiles(Args<T> a)
 {
     using S = TileShape<T, MERGE, K, LMAX>;
-    __shared__ __attribute__((aligned(16))) T s_prod[S::kProd];
+    __shared__ __attribute__((aligned(16))) T s_prod[S::kProd + kSumPad];
     __shared__ int s_rows[2];
     __shared__ int s_desc[6];
     __shared__ ReduceLds<T, S::kWaveCap, S::kBlockCap> L;
@@ -1171,6 +1209,7 @@ template <typename T, int K>
 struct FlatShape {
     static constexpr int kVPT = K / (4 * kBS);                   // 4-nnz vectors per lane
     static constexpr int kRpCap = K + 2;                         // row bounds staged in LDS
+    static constexpr int kRpPer = (kRpCap + kBS - 1) / kBS;      // row_ptr loads per lane
     static constexpr int kWaveCap = K / (kThreadMax + 1) + 1;
     static constexpr int kBlockCap = K / (kWaveMax + 1) + 1;
     static_assert(kVPT * 4 * kBS == K, "K must be a multiple of 1024");
@@ -1183,7 +1222,7 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     constexpr int VPT = S::kVPT;
     constexpr bool DESC = MODE == kFlatDesc;
     using P = acc_t<T>;
-    __shared__ __attribute__((aligned(16))) P s_prod[DESC ? 4 : K];
+    __shared__ __attribute__((aligned(16))) P s_prod[DESC ? 4 : K + kSumPad];
     __shared__ int s_rp[DESC ? 4 : S::kRpCap];
     __shared__ int s_info[4];  // f, row_ptr[f], l, row_ptr[l]
     __shared__ ReduceLds<P, S::kWaveCap, S::kBlockCap> L;
@@ -1200,6 +1239,31 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     const int B = last ? nnz : kb + K;                 // nnz range [kb, B)
     const uint32_t ke = last ? (uint32_t)nnz + 1u : (uint32_t)(kb + K);
 
+    // kFlatMemo: every wave reads the recorded rows itself (a uniform load), so its row_ptr loads go out ahead
+    // of the gathers; reading the map in one lane and row_ptr after the barrier left both latencies after them.
+    int f = 0, rpf = 0, l = 0, rpl = 0;
+    if (MODE == kFlatMemo) {
+        const int2 *mp = reinterpret_cast<const int2 *>(map);
+        const int2 e0 = mp[t], e1 = mp[t + 1];
+        f = e0.x; rpf = e0.y; l = e1.x; rpl = e1.y;
+    }
+    // The rows of the tile, from the first row at or after kb (f), the first at or after ke (l) and their
+    // row_ptr (the FLAT case of make_desc).
+    int head = 0, lo_row = 0, nr = 0, tail = 0;
+    bool ok = true;
+    const auto describe = [&] {
+        head = (f > 0 && rpf > kb) ? 1 : 0;  // row f-1 started before kb and reaches into the tile
+        lo_row = head ? f - 1 : f;
+        nr = l - lo_row;
+        tail = (!last && f < l && rpl > (int)ke) ? 1 : 0;
+        ok = f >= 0 && l >= f && l <= m && lo_row >= 0 && rpf >= kb && rpf <= nnz && rpl <= nnz &&
+             (last || rpl >= (int)ke);
+        if (!ok) {  // row_ptr (or the row map) changed after planning
+            if (tid == 0) atomicOr(a.err, 1);
+            lo_row = 0; nr = 0; tail = 0;
+        }
+    };
+    int rr[S::kRpPer];
     int c[VPT][4];
     T v[VPT][4];
     T xv[VPT][4];
@@ -1216,10 +1280,20 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
                 load4(rc, rv, tid + k * kBS, c[k], v[k]);
             }
         }
-        // The x gathers depend on col only: they are issued before the rows
-        // are known and stay in flight across the row search (or the row map
-        // read) and its barrier, which fences LDS only.  Slots past the tile
-        // read nothing and are never summed.
+        if (MODE == kFlatMemo) {
+            describe();
+            const __amdgpu_buffer_rsrc_t rrp = make_rsrc(a.rp + lo_row, (long long)min(nr + 1, S::kRpCap) * 4);
+#pragma unroll
+            for (int q = 0; q < S::kRpPer; ++q) {
+                rr[q] = 0;
+                if (q * kBS + wave * kWave <= nr)  // wave-uniform
+                    rr[q] = (int)__builtin_amdgcn_raw_buffer_load_b32(rrp, (tid + q * kBS) * 4, 0, 0);
+            }
+        }
+        // The x gathers depend on col only: in the search mode they are issued
+        // before the rows are known and stay in flight across the row search
+        // and its barrier, which fences LDS only.  Slots past the tile read
+        // nothing and are never summed.
         const __amdgpu_buffer_rsrc_t rx = make_rsrc_full(a.x, (long long)a.n * (long long)sizeof(T));
 #pragma unroll
         for (int k = 0; k < VPT; ++k)
@@ -1229,11 +1303,7 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
                                     (T *)nullptr);
     }
     if (MODE == kFlatMemo) {
-        if (tid == 0) {
-            const int2 e0 = reinterpret_cast<const int2 *>(map)[t];
-            const int2 e1 = reinterpret_cast<const int2 *>(map)[t + 1];
-            s_info[0] = e0.x; s_info[1] = e0.y; s_info[2] = e1.x; s_info[3] = e1.y;
-        }
+        // nothing to search
     } else if (wave == 2) {  // f: first row with row_ptr >= kb
         if (MODE == kFlatSearch && a.sched && lane == 0)
             sched_record(a.sched, a.sched_cap, t, kb < nnz ? a.col[kb] : 0, a.n);
@@ -1256,19 +1326,10 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
         }
     }
     if (tid == 0) { L.nw = 0; L.nb = 0; }
-    lds_sync();
-
-    // Descriptor (the FLAT case of make_desc, from the four values).
-    const int f = s_info[0], rpf = s_info[1], l = s_info[2], rpl = s_info[3];
-    const int head = (f > 0 && rpf > kb) ? 1 : 0;  // row f-1 started before kb and reaches into the tile
-    int lo_row = head ? f - 1 : f;
-    int nr = l - lo_row;
-    int tail = (!last && f < l && rpl > (int)ke) ? 1 : 0;
-    const bool ok = f >= 0 && l >= f && l <= m && lo_row >= 0 && rpf >= kb && rpf <= nnz && rpl <= nnz &&
-                    (last || rpl >= (int)ke);
-    if (!ok) {  // row_ptr (or the row map) changed after planning
-        if (tid == 0) atomicOr(a.err, 1);
-        lo_row = 0; nr = 0; tail = 0;
+    if (MODE != kFlatMemo) {
+        lds_sync();
+        f = s_info[0]; rpf = s_info[1]; l = s_info[2]; rpl = s_info[3];
+        describe();
     }
     if (DESC) {
         if (tid == 0) {
@@ -1281,8 +1342,14 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     }
 
     // Row bounds into LDS (global row_ptr is read directly beyond kRpCap).
-    for (int i = tid; i <= nr && i < S::kRpCap; i += kBS)
-        s_rp[i] = a.rp[lo_row + i];
+    if (MODE == kFlatMemo) {
+#pragma unroll
+        for (int q = 0; q < S::kRpPer; ++q)
+            if (tid + q * kBS <= nr && tid + q * kBS < S::kRpCap) s_rp[tid + q * kBS] = rr[q];
+    } else {
+        for (int i = tid; i <= nr && i < S::kRpCap; i += kBS)
+            s_rp[i] = a.rp[lo_row + i];
+    }
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
         if constexpr (strided_layout<T>()) {
@@ -1492,10 +1559,7 @@ __device__ __forceinline__ void rows_sums_staged(const RowsDesc &d, T *s_prod, c
             const int a0 = ra - d.kb;
             const int len = rb - ra;
             if (len <= kThreadMax) {
-                T acc = T(0);
-                for (int j = 0; j < len; ++j)
-                    acc += s_prod[a0 + j];
-                ys[q] = acc;
+                ys[q] = short_row_sum(s_prod + a0, len);
                 mine[q] = true;
             } else if (len <= kWaveMax) {
                 const int j = atomicAdd(&L.nw, 1);
@@ -1509,12 +1573,11 @@ __device__ __forceinline__ void rows_sums_staged(const RowsDesc &d, T *s_prod, c
     lds_sync();
     const int nw = min(L.nw, S::kWaveCap);
     const int nb = min(L.nb, S::kBlockCap);
-    for (int j = wave; j < nw; j += kWaves) {
-        T acc = T(0);
-        for (int q = L.wa[j] + lane; q < L.wb[j]; q += kWave)
-            acc += s_prod[q];
-        acc = wave_sum(acc);
-        if (lane == 0) L.ws[j] = acc;
+    for (int j0 = wave * (kWave / kRowLanes); j0 < nw; j0 += kWaves * (kWave / kRowLanes)) {
+        const int j = j0 + lane / kRowLanes;
+        const int jc = min(j, nw - 1);
+        const T acc = group_row_sum(s_prod, L.wa[jc], j < nw ? L.wb[jc] : 0, lane & (kRowLanes - 1));
+        if (j < nw && (lane & (kRowLanes - 1)) == 0) L.ws[jc] = acc;
     }
     for (int j = 0; j < nb; ++j) {
         T acc = T(0);
@@ -1820,7 +1883,7 @@ __global__ __launch_bounds__(kBS) void k_rows(Args<T> a, int *__restrict__ map, 
     using S = RowsShape<T, K>;
     constexpr int VPT = S::kVPT;
     constexpr bool DESC = MODE == kFlatDesc;
-    __shared__ __attribute__((aligned(16))) acc_t<T> s_prod[DESC ? 4 : S::kProd];
+    __shared__ __attribute__((aligned(16))) acc_t<T> s_prod[DESC ? 4 : S::kProd + kSumPad];
     __shared__ int s_rp[DESC ? 4 : S::kRpCap];
     __shared__ int s_info[4];  // f, row_ptr[f], l, row_ptr[l] (search modes)
     __shared__ RowsReduceLds<acc_t<T>, S::kWaveCap, S::kBlockCap> L;
@@ -2254,10 +2317,7 @@ __device__ __forceinline__ void band_iter(const Args<T> &a, const BandArgs &b, i
             rb = min(max(rb, ra), nq);
         }
         if (rb - ra <= kThreadMax) {
-            P acc = P(0);
-            for (int j = ra; j < rb; ++j)
-                acc += s_prod[j];
-            band_store(ry, i, T(acc));
+            band_store(ry, i, T(short_row_sum(s_prod + ra, rb - ra)));
         } else {
             // disjoint rows of over kThreadMax products: at most kBandList of them (more only with a row_ptr
             // changed after planning, whose rows were clamped above and are reported)
@@ -2279,13 +2339,11 @@ __device__ __forceinline__ void band_iter(const Args<T> &a, const BandArgs &b, i
     if (bad) atomicOr(a.err, 1);
     lds_sync();
     const int nl = min(s_nlist, kBandList);
-    for (int k = wave; k < nl; k += kBandWaves) {
-        const int i = s_list[3 * k], ra = s_list[3 * k + 1], rb = s_list[3 * k + 2];
-        P acc = P(0);
-        for (int j = ra + lane; j < rb; j += kWave)
-            acc += s_prod[j];
-        acc = wave_sum(acc);
-        if (lane == 0) band_store(ry, i, T(acc));
+    for (int k0 = wave * (kWave / kRowLanes); k0 < nl; k0 += kBandWaves * (kWave / kRowLanes)) {
+        const int k = k0 + lane / kRowLanes;
+        const int kc = min(k, nl - 1);
+        const P acc = group_row_sum(s_prod, s_list[3 * kc + 1], k < nl ? s_list[3 * kc + 2] : 0, lane & (kRowLanes - 1));
+        if (k < nl && (lane & (kRowLanes - 1)) == 0) band_store(ry, s_list[3 * kc], T(acc));
     }
 }
 
@@ -2293,7 +2351,7 @@ template <typename T>
 __global__ __launch_bounds__(kBandBS) void k_band(Args<T> a, BandArgs b)
 {
     __shared__ __attribute__((aligned(16))) T s_ring[kBandRing];
-    __shared__ __attribute__((aligned(16))) acc_t<T> s_prod[kBandSlots];
+    __shared__ __attribute__((aligned(16))) acc_t<T> s_prod[kBandSlots + kSumPad];
     __shared__ int s_rp[kBandRp];
     __shared__ int s_list[3 * kBandList];
     __shared__ int s_nlist;
@@ -3159,6 +3217,45 @@ __global__ __launch_bounds__(kBS) void k_fixup(Args<T> a, int K)
         s = wave_sum(s);
         if (lane == 0)
             a.y[rl] = T(a.tail[tl] + s);
+    }
+}
+
+// k_fixup for split-row FLAT plans with a recorded row map: the row leaving
+// tile t and the tile it ends in follow from entries t and t + 1 (the last row
+// starting in tile t is l - 1, which ends at row_ptr[l]), so the partials are
+// read beside the map, not after an owner slot and a row_ptr entry: one memory
+// latency instead of three.  Same sums, in the same order.
+template <typename T>
+__global__ __launch_bounds__(kWave) void k_fixup_map(Args<T> a, const int2 *__restrict__ map, int K)
+{
+    const int lane = threadIdx.x;
+    const long long t = (long long)blockIdx.x * kWave + lane;
+    const bool in = t + 1 < a.ntiles;  // a row leaving the last tile would end past the matrix
+    const int f = in ? map[t].x : 0;
+    const int2 e = in ? map[t + 1] : make_int2(0, 0);
+    const acc_t<T> tail = in ? a.tail[t] : acc_t<T>(0), next = in ? a.head[t + 1] : acc_t<T>(0);
+    bool leaving = in && e.x > f && e.x <= a.m && (long long)e.y > (t + 1) * K;
+    long long tb = leaving ? ((long long)e.y - 1) / K : 0;  // the tile the row ends in
+    if (leaving && tb >= a.ntiles) {  // an entry outside the matrix: report, never dereference
+        atomicOr(a.err, 1);
+        tb = a.ntiles - 1;
+    }
+    if (leaving && tb - t <= kFixSerial) {
+        acc_t<T> s = next;
+        for (long long u = t + 2; u <= tb; ++u)
+            s += a.head[u];
+        a.y[e.x - 1] = T(tail + s);
+        leaving = false;
+    }
+    for (unsigned long long todo = __ballot(leaving); todo; todo &= todo - 1) {  // rows over many tiles: the wave
+        const int k = __ffsll((long long)todo) - 1;
+        const long long t0 = (long long)blockIdx.x * kWave + k;
+        const int r = rlane(e.x, k) - 1, t1 = rlane((int)tb, k);
+        acc_t<T> s = 0;
+        for (long long u = t0 + 1 + lane; u <= t1; u += kWave)
+            s += a.head[u];
+        s = wave_sum(s);
+        if (lane == k) a.y[r] = T(tail + s);
     }
 }
 
@@ -4694,6 +4791,20 @@ int pfk_spmv_fixup(int dtype, int merged_keys, const pfk_spmv_args *a, void *str
 {
     if (a && a->m == 0 && a->nnz == 0) return PF_OK;
     if (!args_ok(a, true) || a->tile <= 0 || !ws_ok(dtype, a, true)) return PF_ERR_INVALID;
+    if (!merged_keys && a->row_map && (a->tile == 1024 || a->tile == 2048)) {  // recorded by the tile kernel before
+        const dim3 mgrid((unsigned)((a->ntiles + kWave - 1) / kWave));
+        const int2 *map = reinterpret_cast<const int2 *>(a->row_map);
+        if (dtype == PF_F64)
+            hipLaunchKernelGGL((k_fixup_map<double>), mgrid, dim3(kWave), 0, S(stream), make_args<double>(a), map, a->tile);
+        else if (dtype == PF_F32)
+            hipLaunchKernelGGL((k_fixup_map<float>), mgrid, dim3(kWave), 0, S(stream), make_args<float>(a), map, a->tile);
+        else if (dtype == PF_F16)
+            hipLaunchKernelGGL((k_fixup_map<half_t>), mgrid, dim3(kWave), 0, S(stream), make_args<half_t>(a), map, a->tile);
+        else
+            return PF_ERR_INVALID;
+        PFK_LAUNCHED("k_fixup_map");
+        return PF_OK;
+    }
     const unsigned grid = (unsigned)((a->ntiles + kBS - 1) / kBS);
     if (dtype == PF_F64) {
         Args<double> r = make_args<double>(a);
