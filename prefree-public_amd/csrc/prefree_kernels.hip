@@ -499,7 +499,9 @@ __device__ __forceinline__ P short_row_sum(const P *s, int len)
 // wave at once; the value, on every lane of the group, is the one wave_sum over
 // lane-strided products gives, bit for bit: lane q's slots q, q + 16, q + 32 and
 // q + 48 stand for those lanes of a wave.  Whole wave active; a == b for a group
-// without a row.
+// without a row.  A wave per row left 16-lane rows' latencies one after another:
+// k_flat on 120,011 rows (8-64 nnz, 120 dense ones, fp32) 40.7 -> 38.1 us per
+// call with the two together, 300,000 rows fp64 137.1 -> 134.3.
 constexpr int kRowLanes = 16;
 
 template <typename P>
@@ -1197,11 +1199,11 @@ template <typename T>
 constexpr bool strided_layout() { return sizeof(T) >= 4; }
 
 // Offset in its tile of element (k, j) of this lane (k < K / 1024, j < 4).
-template <typename T>
+template <typename T, bool STRIDED = strided_layout<T>()>
 __device__ __forceinline__ int tile_elem(int k, int j)
 {
     const int tid = (int)threadIdx.x;
-    return strided_layout<T>() ? k * (4 * kBS) + (tid & ~(kWave - 1)) * 4 + j * kWave + (tid & (kWave - 1))
+    return STRIDED ? k * (4 * kBS) + (tid & ~(kWave - 1)) * 4 + j * kWave + (tid & (kWave - 1))
                                : 4 * (tid + k * kBS) + j;
 }
 
@@ -1215,12 +1217,15 @@ struct FlatShape {
     static_assert(kVPT * 4 * kBS == K, "K must be a multiple of 1024");
 };
 
-template <typename T, int K, int MODE>
+template <typename T, int K, int MODE, bool EARLY_RP = false>
 __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, int *__restrict__ dbg)
 {
     using S = FlatShape<T, K>;
     constexpr int VPT = S::kVPT;
     constexpr bool DESC = MODE == kFlatDesc;
+    // fp16 too where rows are long (not EARLY_RP): a gather over 64 consecutive nnz touches fewer x lines there
+    // (300,000 rows, 300 dense, fp16: 93.5 -> 83.1 us; short power-law rows lose, 42.9 -> 43.8).
+    constexpr bool kStrided = strided_layout<T>() || (MODE == kFlatMemo && !EARLY_RP);
     using P = acc_t<T>;
     __shared__ __attribute__((aligned(16))) P s_prod[DESC ? 4 : K + kSumPad];
     __shared__ int s_rp[DESC ? 4 : S::kRpCap];
@@ -1239,8 +1244,11 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     const int B = last ? nnz : kb + K;                 // nnz range [kb, B)
     const uint32_t ke = last ? (uint32_t)nnz + 1u : (uint32_t)(kb + K);
 
-    // kFlatMemo: every wave reads the recorded rows itself (a uniform load), so its row_ptr loads go out ahead
-    // of the gathers; reading the map in one lane and row_ptr after the barrier left both latencies after them.
+    // kFlatMemo: every wave reads the recorded rows itself (a uniform load), so its row_ptr loads need no barrier:
+    // ahead of the gathers (EARLY_RP) where rows are short and many, right behind them elsewhere, where waiting for
+    // the map first would hold the gathers back (300,000 rows, 300 dense, fp64: 138 us early, 133 late; power law,
+    // 400,001 rows, fp32: 24.1 early, 24.9 late).  One lane reading the map, and row_ptr after a barrier, took 137
+    // and 26.5 us.
     int f = 0, rpf = 0, l = 0, rpl = 0;
     if (MODE == kFlatMemo) {
         const int2 *mp = reinterpret_cast<const int2 *>(map);
@@ -1264,6 +1272,16 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
         }
     };
     int rr[S::kRpPer];
+    const auto rp_loads = [&] {
+        describe();  // waits for the map: not before the gathers unless the loads are
+        const __amdgpu_buffer_rsrc_t rrp = make_rsrc(a.rp + lo_row, (long long)min(nr + 1, S::kRpCap) * 4);
+#pragma unroll
+        for (int q = 0; q < S::kRpPer; ++q) {
+            rr[q] = 0;
+            if (q * kBS + wave * kWave <= nr)  // wave-uniform
+                rr[q] = (int)__builtin_amdgcn_raw_buffer_load_b32(rrp, (tid + q * kBS) * 4, 0, 0);
+        }
+    };
     int c[VPT][4];
     T v[VPT][4];
     T xv[VPT][4];
@@ -1272,24 +1290,15 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
         const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.val + kb, val_range_bytes<T>(B - kb));
 #pragma unroll
         for (int k = 0; k < VPT; ++k) {
-            if constexpr (strided_layout<T>()) {
+            if constexpr (kStrided) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    load1(rc, rv, tile_elem<T>(k, j), c[k][j], v[k][j]);
+                    load1(rc, rv, tile_elem<T, kStrided>(k, j), c[k][j], v[k][j]);
             } else {
                 load4(rc, rv, tid + k * kBS, c[k], v[k]);
             }
         }
-        if (MODE == kFlatMemo) {
-            describe();
-            const __amdgpu_buffer_rsrc_t rrp = make_rsrc(a.rp + lo_row, (long long)min(nr + 1, S::kRpCap) * 4);
-#pragma unroll
-            for (int q = 0; q < S::kRpPer; ++q) {
-                rr[q] = 0;
-                if (q * kBS + wave * kWave <= nr)  // wave-uniform
-                    rr[q] = (int)__builtin_amdgcn_raw_buffer_load_b32(rrp, (tid + q * kBS) * 4, 0, 0);
-            }
-        }
+        if constexpr (MODE == kFlatMemo && EARLY_RP) rp_loads();
         // The x gathers depend on col only: in the search mode they are issued
         // before the rows are known and stay in flight across the row search
         // and its barrier, which fences LDS only.  Slots past the tile read
@@ -1299,8 +1308,9 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
         for (int k = 0; k < VPT; ++k)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                xv[k][j] = buf_load(rx, tile_elem<T>(k, j) < B - kb ? (uint32_t)c[k][j] * (uint32_t)sizeof(T) : kOob,
+                xv[k][j] = buf_load(rx, tile_elem<T, kStrided>(k, j) < B - kb ? (uint32_t)c[k][j] * (uint32_t)sizeof(T) : kOob,
                                     (T *)nullptr);
+        if constexpr (MODE == kFlatMemo && !EARLY_RP) rp_loads();
     }
     if (MODE == kFlatMemo) {
         // nothing to search
@@ -1352,10 +1362,10 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     }
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-        if constexpr (strided_layout<T>()) {
+        if constexpr (kStrided) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                s_prod[tile_elem<T>(k, j)] = P(v[k][j]) * P(xv[k][j]);
+                s_prod[tile_elem<T, kStrided>(k, j)] = P(v[k][j]) * P(xv[k][j]);
         } else {
             P p[4];
 #pragma unroll
@@ -2461,6 +2471,7 @@ struct DenseShape {
     static_assert(kW == PFK_DENSE_WINDOW(sizeof(T) == 8 ? PF_F64 : sizeof(T) == 4 ? PF_F32 : PF_F16),
                   "window of the C ABI");
 };
+
 
 struct DenseArgs {
     const int *__restrict__ rows;  // dense rows, ascending
@@ -4426,6 +4437,9 @@ int launch_flat(const pfk_spmv_args *a, int *dbg, void *stream)
     }
     if (dbg)
         hipLaunchKernelGGL((k_flat<T, K, kFlatDesc>), dim3((unsigned)grid), dim3(kBS), 0, S(stream), r, nullptr, dbg);
+    else if (a->row_map && a->map_ready && (long long)a->nnz < 16LL * a->m)  // many rows per tile
+        hipLaunchKernelGGL((k_flat<T, K, kFlatMemo, true>), dim3((unsigned)(a->sched ? a->sched_cap * kXcds : grid)),
+                           dim3(kBS), 0, S(stream), r, a->row_map, nullptr);
     else if (a->row_map && a->map_ready)
         hipLaunchKernelGGL((k_flat<T, K, kFlatMemo>), dim3((unsigned)(a->sched ? a->sched_cap * kXcds : grid)),
                            dim3(kBS), 0, S(stream), r, a->row_map, nullptr);
