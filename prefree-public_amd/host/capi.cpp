@@ -675,14 +675,11 @@ int plan_add_split(pf_plan *p)
     return PF_OK;
 }
 
-// Dense-row threshold of a hybrid plan: a power of two at least 4096 and at
-// least 256 n / W, so that a dense row averages 256 or more nnz per x window.
+// Dense-row threshold of a hybrid plan: at least 4096 nnz and at least 256 n / W, so that a dense row averages
+// 256 or more nnz per x window.
 long long dense_min(long long n, int dtype)
 {
-    const long long want = std::max(4096LL, (256LL * n + PFK_DENSE_WINDOW(dtype) - 1) / PFK_DENSE_WINDOW(dtype));
-    long long t = 4096;
-    while (t < want) t <<= 1;
-    return t;
+    return std::max(4096LL, (256LL * n + PFK_DENSE_WINDOW(dtype) - 1) / PFK_DENSE_WINDOW(dtype));
 }
 
 // Rows of at least 2^j nnz, from the log2 histogram (bucket k: 2^(k-1) <= len < 2^k).
@@ -732,8 +729,8 @@ bool hybrid_candidate(const pf_row_stats &s, long long n, int dtype, const pf_pl
         !uses_row_map(info.variant, info.tile) || s.n_long_rows < 1)
         return false;
     const long long t = dense_min(n, dtype);
-    int j = 0;
-    while ((1LL << j) < t) ++j;
+    int j = 0;  // the histogram counts rows by power of two: the one at or below the threshold
+    while ((2LL << j) <= t) ++j;
     return rows_at_least_pow2(s, j) == s.n_long_rows || n * value_bytes(dtype) > kXcdL2Bytes;
 }
 
