@@ -54,6 +54,7 @@ constexpr long long kXcdL2Bytes = 4LL << 20;  // MI355X: 4 MB of L2 per XCD
 // AUTO's row groups: at most 2^18 rows whose values and columns fit the 256 MB MALL
 constexpr long long kRowGroupRowsMax = 1LL << 18;
 constexpr long long kRowGroupBytesMax = 256LL << 20;
+constexpr long long kRowGroupWideBytesMax = 64LL << 20;  // over 2^18 rows (see auto_choice)
 constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
 
 // Tiles per XCD list of an x-window schedule: an even share plus 2% slack.
@@ -314,8 +315,16 @@ int row_group_lanes(const pf_row_stats &s)
 //     row_group_lanes lanes per row (k_vector: no tiles, no workspace, one
 //     launch; fp64 C1 1.9 us per SpMV in a graph against 3.5 for 1024-nnz
 //     tiles; 131072 rows of 32 nnz 24.8 against 28.7; 262144 x 64 86 against
-//     99; 262144 x 128, 403 MB, 239 against 192 for 2048-nnz tiles; 393216 x
-//     8, 23.8 for 1024-nnz tiles against 24.3 for the best row groups);
+//     99; 262144 x 128, 403 MB, 239 against 192 for 2048-nnz tiles);
+//   * more rows, none longer than 64, of 7 to 16 nnz on average, values and
+//     columns within 64 MB: row groups too.  A tile's barriers and LDS round
+//     trip hold its gathers back where a call is little more than one round of
+//     tiles; 300007 rows of 16 random columns, fp64 34.3 us for 1024-nnz tiles,
+//     28.6 for 8 lanes per row, fp32 29.0 and 24.7, fp16 25.8 and 23.1; rows of
+//     8: 20.7 and 16.4 (fp64).  The lines: 16-nnz rows over 115 MB (600000,
+//     fp64) take 82 us against 71 for tiles, 77 MB (fp32) 48.4 against 51.3;
+//     24-nnz rows 49.7 against 48.3 and 27-point stencils 31.3 against 27.4
+//     (300000, fp64); 5-point grids take tiles at every size over 2^18 rows;
 //   * no row longer than PFK_ALIGN_ROW_MAX, or fp16 values (FLAT only): FLAT
 //     (1024 nnz per tile for fp64, 2048 for fp32 / fp16 or for rows of under
 //     4 nnz on average), row-aligned when the rows fit: one launch per call;
@@ -336,8 +345,10 @@ Choice auto_choice(const pf_row_stats &s, int dtype)
     if (table_choice(s, dtype, c)) return c;
     const long long m = s.m, nnz = s.nnz;
     c.variant = PF_FLAT;
-    if (s.max_row_len <= PFK_ALIGN_ROW_MAX && m > 0 && m <= kRowGroupRowsMax &&
-        nnz * (value_bytes(dtype) + 4) <= kRowGroupBytesMax) {
+    const long long stream = nnz * (value_bytes(dtype) + 4);
+    const bool few = m <= kRowGroupRowsMax && stream <= kRowGroupBytesMax;
+    const bool middling = s.max_row_len <= 64 && nnz >= 7 * m && nnz <= 16 * m + m / 2 && stream <= kRowGroupWideBytesMax;
+    if (s.max_row_len <= PFK_ALIGN_ROW_MAX && m > 0 && (few || middling)) {
         c.tile = row_group_lanes(s);
         return c;
     }

@@ -92,3 +92,29 @@ def test_row_groups_at_the_rule_bounds():
         if want_groups:
             assert info["tile"] == 32, info
         assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"bounds {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("extra,longest,groups", [(0, 64, True), (-1, 64, False), (0, 65, False)])
+def test_auto_over_2_18_rows_of_middling_length(extra, longest, groups, dtype):
+    """One row more than 2^18, 7 nnz per row on average: row groups at the rule's lower edge and at the longest row
+    it takes, tiles one nnz below the one or above the other; ragged rows, empty ones among them, against the oracle."""
+    rng = np.random.default_rng(7)
+    m = (1 << 18) + 1
+    lens = rng.integers(0, 14, m)
+    lens[rng.integers(0, m)] = 0
+    lens[m - 1] = longest
+    short = 7 * m + extra - int(lens.sum())  # the rest of the nnz, over rows that stay under 32
+    at = rng.choice(m - 1, abs(short), replace=False)
+    if short < 0:
+        at = np.flatnonzero(lens[:m - 1] > 0)[:-short]
+    lens[at] += 1 if short > 0 else -1
+    assert lens.sum() == 7 * m + extra and lens.max() == longest and lens.min() == 0
+    rp = np.zeros(m + 1, dtype=np.int64)
+    np.cumsum(lens, out=rp[1:])
+    rp = rp.astype(np.int32)
+    col = rng.integers(0, 60000, int(rp[-1])).astype(np.int32)
+    val, x = oracle.initvec(len(col), NP[dtype]), oracle.initvec(60000, NP[dtype])
+    y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
+    assert (info["variant_name"], info["tile"] <= 32) == ("flat", groups), info
+    assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{extra} {longest} {dtype}")
