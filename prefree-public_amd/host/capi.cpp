@@ -1573,9 +1573,60 @@ int pf_plan_destroy(pf_plan *plan)
     return st == PF_OK ? PF_OK : from_kernel_layer(st, "free workspace");
 }
 
+// One-shot y = A x with its statistics and workspace in the device's scratch array, under the lock the caller holds
+// (`scratch_lock`), until the stream is synchronised.
+static int spmv_in_scratch(void *scr, size_t scr_bytes, const int *d_row_ptr, const int *d_col, const void *d_val,
+                           const void *d_x, void *d_y, int m, int n, int nnz, int dtype, int variant, void *stream)
+{
+    pf_plan p;  // on the stack: no allocation of any kind
+    p.m = m;
+    p.n = n;
+    p.nnz = nnz;
+    int st = stats_via(static_cast<unsigned long long *>(scr), d_row_ptr, d_col, m, n, nnz, &p.stats, stream);
+    if (st != PF_OK) return st;
+    st = check_csr_stats(p.stats, nnz);
+    if (st != PF_OK) return st;
+    st = plan_info(p.stats, n, dtype, variant, 0, &p.info);
+    if (st != PF_OK) return st;
+    if (p.info.workspace_bytes > scr_bytes - kNoallocStatsBytes)
+        return fail(PF_ERR_UNSUPPORTED, "pf_spmv_noalloc: the workspace needs " + std::to_string(p.info.workspace_bytes) +
+                                            " bytes, the scratch holds " +
+                                            std::to_string(scr_bytes - kNoallocStatsBytes) + "; use pf_spmv");
+    plan_carve(&p, static_cast<char *>(scr) + kNoallocStatsBytes);
+    // row-aligned tiles split no row, so no owner slot is read: the error flag alone starts cleared
+    st = p.info.row_aligned ? pfk_fill_zero(p.err, 256, stream) : plan_init(&p, d_row_ptr, stream);
+    if (st != PF_OK) return from_kernel_layer(st, "scratch workspace init");
+    st = pf_plan_execute(&p, d_row_ptr, d_col, d_val, d_x, d_y, stream);
+    if (st == PF_OK) st = pf_plan_check(&p, stream);  // synchronises: the scratch is free again on return
+    else pfk_stream_sync(stream);
+    return st;
+}
+
+// A one-shot call's plan lives for one product, so it is made in the device's scratch array where that is free and
+// large enough: no hipMalloc, hipFree, events or planning waits beyond the statistics' one.  us per call, with a
+// plan of its own -> in the scratch: 1448^2 5-point grid fp64 190 -> 107, 4096 rows of 16 100 -> 62, 2M power-law
+// rows 1012 -> 336 (no hybrid tables for one product), 20M rows of 2.5 (50M nnz) 532 -> 532.  Above kScratchNnz the
+// tables pay even once or the workspace may not fit; those calls, explicit variants, incomplete arguments (for their
+// error) and calls that find another thread in the scratch make a plan.
+constexpr long long kScratchNnz = 64LL << 20;
+
 int pf_spmv(const int *d_row_ptr, const int *d_col, const void *d_val, const void *d_x, void *d_y, int m, int n,
             int nnz, int dtype, int variant, void *stream)
 {
+    int dev = 0;
+    void *scr = nullptr;
+    size_t scr_bytes = 0;
+    if (variant == PF_AUTO && m > 0 && nnz > 0 && nnz <= kScratchNnz && d_row_ptr && d_col && d_val && d_x && d_y &&
+        check_matrix_args(d_row_ptr, d_col, m, n, nnz, dtype, variant) == PF_OK && aligned16(d_val) &&
+        pfk_get_device(&dev) == PF_OK && dev >= 0 && dev < kNoallocDevices && pfk_scratch(&scr, &scr_bytes) == PF_OK) {
+        std::unique_lock<std::mutex> lock(g_noalloc_mu[dev], std::try_to_lock);
+        if (lock.owns_lock()) {
+            warm_queues();
+            const int st = spmv_in_scratch(scr, scr_bytes, d_row_ptr, d_col, d_val, d_x, d_y, m, n, nnz, dtype, variant,
+                                           stream);
+            if (st != PF_ERR_UNSUPPORTED) return st;
+        }
+    }
     pf_plan *p = nullptr;
     int st = pf_plan_create(&p, d_row_ptr, d_col, m, n, nnz, dtype, variant, stream);
     if (st != PF_OK) return st;
@@ -1613,27 +1664,8 @@ int pf_spmv_noalloc(const int *d_row_ptr, const int *d_col, const void *d_val, c
     int dev = 0;
     PF_TRY(pfk_get_device(&dev), "current device");
     if (dev < 0 || dev >= kNoallocDevices) return fail(PF_ERR_UNSUPPORTED, "device index beyond the scratch table");
-    std::lock_guard<std::mutex> scratch_lock(g_noalloc_mu[dev]);  // held until the stream is synchronised below
-    pf_plan p;  // on the stack: no allocation of any kind
-    p.m = m;
-    p.n = n;
-    p.nnz = nnz;
-    st = stats_via(static_cast<unsigned long long *>(scr), d_row_ptr, d_col, m, n, nnz, &p.stats, stream);
-    if (st != PF_OK) return st;
-    st = check_csr_stats(p.stats, nnz);
-    if (st != PF_OK) return st;
-    st = plan_info(p.stats, n, dtype, variant, 0, &p.info);
-    if (st != PF_OK) return st;
-    if (p.info.workspace_bytes > scr_bytes - kNoallocStatsBytes)
-        return fail(PF_ERR_UNSUPPORTED, "pf_spmv_noalloc: the workspace needs " + std::to_string(p.info.workspace_bytes) +
-                                            " bytes, the scratch holds " +
-                                            std::to_string(scr_bytes - kNoallocStatsBytes) + "; use pf_spmv");
-    plan_carve(&p, static_cast<char *>(scr) + kNoallocStatsBytes);
-    st = plan_init(&p, d_row_ptr, stream);
-    if (st != PF_OK) return from_kernel_layer(st, "scratch workspace init");
-    st = pf_plan_execute(&p, d_row_ptr, d_col, d_val, d_x, d_y, stream);
-    if (st == PF_OK) st = pf_plan_check(&p, stream);  // synchronises: the scratch is free again on return
-    return st;
+    std::lock_guard<std::mutex> scratch_lock(g_noalloc_mu[dev]);  // held until the stream is synchronised
+    return spmv_in_scratch(scr, scr_bytes, d_row_ptr, d_col, d_val, d_x, d_y, m, n, nnz, dtype, variant, stream);
 }
 
 int pf_set_tuning_table(const char *path)
