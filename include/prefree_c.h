@@ -252,7 +252,8 @@ int pf_plan_autotune(pf_plan *plan, const int *d_row_ptr, const int *d_col, cons
  * per row on average), regular (no row over 256 nnz), skewed (longer rows, under 16 nnz per row on
  * average), dense (longer rows, 16 or more on average) — or any.  The first row whose dtype and row
  * class match and whose bound exceeds the matrix's nnz decides (run 0: the built-in run rule; ladder
- * 0: the default ladder; hybrid 0: a FLAT plan stays split-row even with dense rows).  Rows of the
+ * 0: the default ladder; hybrid 0: a FLAT plan stays split-row even with dense rows; flat 16 and a matrix with
+ * rows over 256 nnz: row groups beside long rows, a workgroup each, where they pay, and the next row elsewhere).  Rows of the
  * older form <class> <nnz_upper> <dtype> <variant> <tile> <run> <keep> match any row class.
  * NULL clears the table.  Without a call, the table named by $PREFREE_TUNING_TABLE is read once (an
  * empty value: none) or, when that is unset, tune/mi355x_tuning_table.txt beside the lib/ directory

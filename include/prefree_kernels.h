@@ -142,6 +142,10 @@ typedef struct pfk_spmv_args {
 /* nnz per long-row tile of a hybrid plan in long mode. */
 #define PFK_LONG_TILE 1024
 
+/* Row groups beside long rows (pfk_spmv_flat, tile = PFK_VECTOR_LONG_LANES, n_dense > 0): dense_rows lists the rows
+ * over PFK_ALIGN_ROW_MAX nnz, each once; a workgroup sums each of them whole and the row groups the others. */
+#define PFK_VECTOR_LONG_LANES 16
+
 /* Bytes of one split-row partial (head / tail slot): fp32 in the fp16 mode. */
 #define PFK_SLOT_BYTES(dtype) ((dtype) == 0 ? 8 : 4)
 

@@ -3361,6 +3361,104 @@ __global__ __launch_bounds__(kBS) void k_vector(Args<T> a)
     if (q == 0) a.y[g] = T(s);
 }
 
+// ---- k_vector_long: row groups beside long rows ---------------------------
+//
+// k_vector for matrices with a few rows over kAlignRowMax nnz (the plan's list):
+// workgroup i < nlong sums the i-th of them whole, the others the row groups,
+// which leave those rows out.  One launch, no barrier among the groups, no
+// partial sums and no combine: a long row keeps its workgroup of 1024 lanes for
+// some microseconds (60,000 nnz: eight batches) beside the others' gathers.
+// us per call against split-row tiles and their combine: 20,011 rows of 8-64
+// nnz and 20 of 1,000-10,000, fp64 11.6 -> 8.0, fp32 10.2 -> 5.8; 120,011 rows,
+// 120 long ones, fp64 46.1 -> 39.3, fp32 36.6 -> 30.3, fp16 33.2 -> 26.5.  It
+// is bound by its gathers' L2 lines and, below 40,000 rows, by three memory
+// latencies.  Long rows stream kVecU elements
+// per lane and batch, the next batch's columns and values in flight while a
+// batch's x arrives (two batches by name, so that no register with a load in
+// flight is copied); lane partials, then the wave's tree, then the waves in
+// order.
+constexpr int kVecBS = 1024;
+constexpr int kVecU = 8;
+
+template <typename T, int L>
+__global__ __launch_bounds__(kVecBS) void k_vector_long(Args<T> a, const int *__restrict__ rows, int nlong)
+{
+    using P = acc_t<T>;
+    __shared__ P s_red[kVecBS / kWave];
+    const int tid = threadIdx.x;
+    const int nnz = a.nnz;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc_full(a.x, (long long)a.n * (long long)sizeof(T));
+    if ((int)blockIdx.x < nlong) {
+        const int r = min(max(uni(rows[blockIdx.x]), 0), a.m - 1);
+        const int r0 = min(max(uni(a.rp[r]), 0), nnz);
+        const int r1 = min(max(uni(a.rp[r + 1]), r0), nnz);
+        if (r1 - r0 <= kAlignRowMax) {  // row_ptr changed after planning: the row groups sum this row
+            if (tid == 0) atomicOr(a.err, 1);
+            return;
+        }
+        const int ra = r0 & ~(kWave - 1);  // whole lines per load; the nnz before the row add nothing
+        const int lead = r0 - ra, len = r1 - ra;
+        const __amdgpu_buffer_rsrc_t rc = make_rsrc(a.col + ra, (long long)len * 4);
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(a.val + ra, val_range_bytes<T>(len));
+        int cA[kVecU], cB[kVecU];
+        T vA[kVecU], vB[kVecU];
+        P acc = P(0);
+        const auto issue = [&](int b, int (&c)[kVecU], T (&v)[kVecU]) {
+#pragma unroll
+            for (int u = 0; u < kVecU; ++u) load1(rc, rv, b + u * kVecBS + tid, c[u], v[u]);
+        };
+        const auto consume = [&](int b, const int (&c)[kVecU], const T (&v)[kVecU], int next, int (&cn)[kVecU], T (&vn)[kVecU]) {
+            T xv[kVecU];
+#pragma unroll
+            for (int u = 0; u < kVecU; ++u) {
+                const int q = b + u * kVecBS + tid;
+                xv[u] = buf_load(rx, q >= lead && q < len ? (uint32_t)c[u] * (uint32_t)sizeof(T) : kOob, (T *)nullptr);
+            }
+            if (next < len) issue(next, cn, vn);
+            P p[kVecU];  // a batch's products as a tree, then to the lane's sum: 8 roundings in a row where 60 were
+#pragma unroll
+            for (int u = 0; u < kVecU; ++u) {
+                const int q = b + u * kVecBS + tid;
+                p[u] = q >= lead && q < len ? P(v[u]) * P(xv[u]) : P(0);
+            }
+#pragma unroll
+            for (int h = kVecU / 2; h > 0; h /= 2)
+#pragma unroll
+                for (int u = 0; u < h; ++u) p[u] += p[u + h];
+            acc += p[0];
+        };
+        constexpr int kB = kVecU * kVecBS;
+        issue(0, cA, vA);
+        for (int b = 0; b < len; b += 2 * kB) {
+            consume(b, cA, vA, b + kB, cB, vB);
+            if (b + kB < len) consume(b + kB, cB, vB, b + 2 * kB, cA, vA);
+        }
+        acc = wave_sum(acc);
+        if ((tid & (kWave - 1)) == 0) s_red[tid / kWave] = acc;
+        lds_sync();
+        if (tid == 0) {
+            P tot = s_red[0];
+#pragma unroll
+            for (int w = 1; w < kVecBS / kWave; ++w) tot += s_red[w];
+            a.y[r] = T(tot);
+        }
+        return;
+    }
+    const long long g = ((long long)(blockIdx.x - nlong) * kVecBS + tid) / L;
+    const int q = tid & (L - 1);
+    if (g >= a.m)
+        return;  // whole groups
+    const int r0 = min(max(a.rp[g], 0), nnz);
+    const int r1 = min(max(a.rp[g + 1], r0), nnz);
+    const bool apart = r1 - r0 > kAlignRowMax;
+    P s = P(0);
+    if (!apart)
+        for (int j = r0 + q; j < r1; j += L)
+            s += P(a.val[j]) * P(buf_load(rx, (uint32_t)a.col[j] * (uint32_t)sizeof(T), (T *)nullptr));
+    s = group_sum<L>(s);
+    if (q == 0 && !apart) a.y[g] = T(s);
+}
+
 // ---- k_prefree: the reference kernel's algorithm on wave64 -----------------
 
 constexpr int kPfBS = 128;  // preFreeSpMV.cu:583
@@ -4460,6 +4558,18 @@ int launch_vector(const pfk_spmv_args *a, void *stream)
     if (grid < 1 || grid > 0x7FFFFFFFLL) {
         snprintf(g_err, sizeof g_err, "row groups: %lld workgroups", grid);
         return PF_ERR_UNSUPPORTED;
+    }
+    if (a->n_dense > 0) {  // long rows beside the row groups
+        if (a->tile != PFK_VECTOR_LONG_LANES || !a->dense_rows) {
+            snprintf(g_err, sizeof g_err, "row groups beside long rows: %d lanes per row, and the rows' list",
+                     PFK_VECTOR_LONG_LANES);
+            return PF_ERR_INVALID;
+        }
+        const long long lgrid = ((long long)a->m * a->tile + kVecBS - 1) / kVecBS + a->n_dense;
+        hipLaunchKernelGGL((k_vector_long<T, PFK_VECTOR_LONG_LANES>), dim3((unsigned)lgrid), dim3(kVecBS), 0, S(stream),
+                           r, a->dense_rows, a->n_dense);
+        PFK_LAUNCHED("k_vector_long");
+        return PF_OK;
     }
     switch (a->tile) {
     case 2: hipLaunchKernelGGL((k_vector<T, 2>), dim3((unsigned)grid), dim3(kBS), 0, S(stream), r); break;

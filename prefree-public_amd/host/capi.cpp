@@ -55,6 +55,7 @@ constexpr long long kXcdL2Bytes = 4LL << 20;  // MI355X: 4 MB of L2 per XCD
 constexpr long long kRowGroupRowsMax = 1LL << 18;
 constexpr long long kRowGroupBytesMax = 256LL << 20;
 constexpr long long kRowGroupWideBytesMax = 64LL << 20;  // over 2^18 rows (see auto_choice)
+constexpr long long kVectorLongBytesMax = 128LL << 20;  // see vector_long_rule
 constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
 
 // Tiles per XCD list of an x-window schedule: an even share plus 2% slack.
@@ -124,7 +125,9 @@ int choose_run(int tile, long long ntiles, long long resident)
 // One row per (size class, row-length class, value type): nnz below
 // `nnz_upper` (-1: no bound) and the matrix's row-length class select
 // (variant, tile, run_tiles, keep_cached, ladder, hybrid), or variant "auto"
-// (tile 0): the built-in rules.  The row-length
+// (tile 0): the built-in rules.  A FLAT row of 16 lanes means, for a matrix with
+// long rows, row groups beside them where vector_long_rule takes them, and the
+// next row elsewhere.  The row-length
 // classes are the cuts of the built-in rules below: "short" (every row <= 256
 // nnz, under 4 nnz per row on average), "regular" (every row <= 256 nnz),
 // "skewed" (longer rows, under 16 nnz per row on average), "dense" (longer
@@ -261,10 +264,12 @@ bool tile_supported(int variant, int dtype, int tile);
 
 // Decision of PF_AUTO: variant and tile, plus the run length and cache
 // policy when a tuning-table row fixes them (run 0 / keep -1: not fixed), the
-// PREFREE ladder (0: the default) and whether FLAT may turn hybrid.
+// PREFREE ladder (0: the default), whether FLAT may turn hybrid and whether
+// row groups beside long rows may take its place.
 struct Choice {
     int variant = PF_ADAPTIVE, tile = 0, run = 0, keep = -1, ladder = 0;
     bool hybrid = true;
+    bool beside = true;  // row groups beside long rows, where vector_long_rule takes them
 };
 
 bool table_choice(const pf_row_stats &s, int dtype, Choice &c)
@@ -272,17 +277,23 @@ bool table_choice(const pf_row_stats &s, int dtype, Choice &c)
     std::lock_guard<std::mutex> lock(g_table_mu);
     table_init_locked();
     const int rc = row_class(s);
+    bool beside = false;
     for (const TableRow &r : g_table) {
         if (r.dtype != dtype || (r.nnz_upper >= 0 && s.nnz >= r.nnz_upper)) continue;
         if (r.rows != kRowsAny && r.rows != rc) continue;
         if (r.variant == PF_AUTO) return false;  // this class keeps the built-in rules
         if (!tile_supported(r.variant, dtype, r.tile)) continue;
+        if (r.variant == PF_FLAT && r.tile == PFK_VECTOR_LONG_LANES && s.n_long_rows > 0) {
+            beside = true;  // with long rows: beside them where vector_long_rule says so, else the next row
+            continue;
+        }
         c.variant = r.variant;
         c.tile = r.tile;
         c.run = r.run;
         c.keep = r.keep;
         c.ladder = r.ladder;
         c.hybrid = r.hybrid != 0;
+        c.beside = beside;
         return true;
     }
     return false;
@@ -537,6 +548,9 @@ struct pf_plan {
     int *long_tiles = nullptr, *long_deal = nullptr, *long_row_tiles = nullptr;
     void *long_part = nullptr;
     size_t long_tiles_bytes = 0, long_deal_bytes = 0, long_row_tiles_bytes = 0, long_part_bytes = 0;
+    // row groups beside long rows: the rows over PFK_ALIGN_ROW_MAX nnz, longest first
+    int *long_rows = nullptr;  // its own allocation
+    int n_long_rows = 0;
     // the runs' stream beside the caller's, and the events that fork and join it (see pfk_spmv_args)
     void *aux_stream = nullptr, *ev_fork = nullptr, *ev_join = nullptr;
 };
@@ -547,15 +561,18 @@ namespace {
 // (host only, apart from occupancy queries): variant and tile (PF_AUTO
 // resolved), run length, x windows, workspace size.
 // `allow_hybrid` (optional) tells whether a FLAT plan of PF_AUTO may turn
-// hybrid: always, unless a tuning-table row says otherwise.
+// hybrid: always, unless a tuning-table row says otherwise; `allow_beside`
+// whether row groups beside long rows may replace it.
 int plan_info(const pf_row_stats &s, int n, int dtype, int variant, int tile, pf_plan_info *out,
-              bool *allow_hybrid = nullptr)
+              bool *allow_hybrid = nullptr, bool *allow_beside = nullptr)
 {
     Choice c;
     if (allow_hybrid) *allow_hybrid = true;
+    if (allow_beside) *allow_beside = false;
     if (variant == PF_AUTO) {  // an explicit tile is kept only if the chosen variant has it
         c = auto_choice(s, dtype);
         if (allow_hybrid) *allow_hybrid = c.hybrid;
+        if (allow_beside) *allow_beside = c.beside;
         variant = c.variant;
         if (tile <= 0 || !tile_supported(variant, dtype, tile)) tile = c.tile;
     }
@@ -964,6 +981,46 @@ int try_hybrid(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream,
     return PF_OK;
 }
 
+// PF_AUTO: row groups beside long rows (k_vector_long), for a few long rows among short ones of middling length,
+// where the table or the rules would cut every row at tile edges.  The short rows hold 12 nnz or more on average
+// and at most 128 (8 passes of a group), the long rows 1024 or more on average and at most 2^16, values and
+// columns are within 128 MB and x within one XCD's L2.  Measured, us per call, against the tiles: rows of 8-64 nnz
+// with a thousandth of long ones, fp64: 20,011 rows 8.0 against 11.6, 60,000 rows 20 against 25, 120,011 (99 MB)
+// 39 against 46, 200,001 (221 MB) 83 against 79; fp32: 120,011 rows 30 against 37, 200,001 (147 MB) 58 against 60,
+// 300,000 (280 MB) 107 against 96.  Short rows of 4 nnz (power law) take 55 against 24.
+bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanScan *scan)
+{
+    if (!scan || !scan->list || s.n_long_rows < 1 || scan->listed != s.n_long_rows || scan->host_n != scan->listed)
+        return false;
+    long long long_nnz = 0;
+    for (long long k = 0; k < scan->host_n; ++k)
+        long_nnz += scan->host[(size_t)(4 * k + 2)] - (long long)scan->host[(size_t)(4 * k + 1)];
+    const long long short_nnz = s.nnz - long_nnz, short_rows = s.m - s.n_long_rows;
+    return s.max_row_len <= (1LL << 16) && long_nnz >= 1024 * s.n_long_rows && s.max_short_row_len <= 128 &&
+           short_nnz >= 12 * short_rows && s.nnz * (value_bytes(dtype) + 4) <= kVectorLongBytesMax &&
+           n * value_bytes(dtype) <= kXcdL2Bytes;
+}
+
+// The list of a row-groups-beside-long-rows plan on the device, longest row first (the long rows start with the
+// call).  Synchronises `stream`.
+int add_long_rows(pf_plan *p, const PlanScan &scan, void *stream)
+{
+    const size_t count = (size_t)scan.host_n;
+    std::vector<int> order(count), rows(count);
+    for (size_t k = 0; k < count; ++k) order[k] = (int)k;
+    const auto len = [&](int k) { return scan.host[(size_t)(4 * k + 2)] - scan.host[(size_t)(4 * k + 1)]; };
+    std::sort(order.begin(), order.end(), [&](int x, int y) {
+        return len(x) != len(y) ? len(x) > len(y) : scan.host[(size_t)(4 * x)] < scan.host[(size_t)(4 * y)];
+    });
+    for (size_t k = 0; k < count; ++k) rows[k] = scan.host[(size_t)(4 * order[k])];
+    PF_TRY(pfk_malloc(reinterpret_cast<void **>(&p->long_rows), count * sizeof(int)), "long-row list");
+    int st = pfk_memcpy_h2d(p->long_rows, rows.data(), count * sizeof(int), stream);
+    if (st == PF_OK) st = pfk_stream_sync(stream);
+    if (st != PF_OK) return from_kernel_layer(st, "long-row list");
+    p->n_long_rows = (int)count;
+    return PF_OK;
+}
+
 // The band kernel for a row-aligned plan: measures (on a sample of the rows)
 // how many columns lie within +-w of their row (w = 64 << i) and keeps the
 // smallest w that holds 85% of the nnz and, with two steps' rows, fits the
@@ -1009,11 +1066,19 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
                void *stream, pf_plan **plan, const int *d_col = nullptr, const PlanScan *scan = nullptr,
                PlanTimer *timer = nullptr)
 {
-    bool allow_hybrid = true;
+    bool allow_hybrid = true, allow_beside = false;
     pf_plan_info info;
-    const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid);
-    const bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && allow_hybrid;
+    const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid, &allow_beside);
+    bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && allow_hybrid;
     if (st != PF_OK) return st;
+    bool beside = false;  // row groups beside long rows
+    if (allow_beside && tile <= 0 && !(want_hybrid && hybrid_candidate(s, n, dtype, info, d_col)) &&
+        vector_long_rule(s, n, dtype, scan)) {
+        const int st2 = finish_info(s, dtype, PF_FLAT, PFK_VECTOR_LONG_LANES, &info);
+        if (st2 != PF_OK) return st2;
+        beside = true;
+        want_hybrid = false;
+    }
     pf_plan *p = new pf_plan();
     p->m = m;
     p->n = n;
@@ -1039,6 +1104,15 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         rc = plan_init(p, d_row_ptr, stream);
         if (rc == PF_OK) rc = pfk_stream_sync(stream);
         if (rc == PF_OK && timer) timer->stop(stream);
+    }
+    if (rc == PF_OK && beside) {
+        rc = add_long_rows(p, *scan, stream);
+        if (rc != PF_OK) {
+            pfk_free(p->long_rows);
+            pfk_free(p->ws);
+            delete p;
+            return rc;
+        }
     }
     if (rc == PF_OK && d_col && !candidate) rc = try_band(p, d_row_ptr, d_col, stream, timer);
     if (rc == PF_OK && candidate) {
@@ -1459,6 +1533,8 @@ int pf_plan_execute(pf_plan *plan, const int *d_row_ptr, const int *d_col, const
     // no row of a row-aligned tile is longer than this (longer rows take other plans), so the tile kernel can
     // load a tile's overflow with its nominal range
     a.ovf_cap = plan->info.row_aligned ? (int)std::min<long long>(PFK_ALIGN_ROW_MAX, plan->stats.max_row_len) : 0;
+    a.dense_rows = plan->long_rows;
+    a.n_dense = plan->n_long_rows;
     a.band_w = a.row_map ? plan->info.band_w : 0;  // used once the row map is recorded; never without one
     const int dt = plan->info.dtype;
     if (plan->hybrid) {
@@ -1561,6 +1637,10 @@ int pf_plan_destroy(pf_plan *plan)
         pfk_stream_destroy(plan->aux_stream);
     }
     int st = pfk_free(plan->ws);
+    if (plan->long_rows) {
+        const int st2 = pfk_free(plan->long_rows);
+        if (st == PF_OK) st = st2;
+    }
     if (plan->ws_split) {
         const int st2 = pfk_free(plan->ws_split);
         if (st == PF_OK) st = st2;

@@ -1,0 +1,121 @@
+"""Row groups beside long rows: AUTO's plan for a few long rows among short ones of middling length, against the
+oracle, at the edges of its rule and of its kernel (batches of 8192 nnz, rows that start inside a line, long rows
+first, last and next to each other)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import prefree_amd as pf
+from csr_cases import csr_from_lengths
+from gpu_util import DEV, NP, TORCH, assert_parity, dev, gpu_spmv, kat_exact_possible
+
+pytestmark = pytest.mark.gpu
+
+# lengths of the long rows, and where they stand among 3001 short rows of 0-40 nnz (an odd count, so that they
+# start anywhere in a line)
+LONG = {
+    "one": [(1500, 3000)],
+    "first_and_last": [(0, 1024), (3000, 1025)],
+    "adjacent": [(7, 8191), (8, 8192), (9, 8193)],
+    "largest": [(100, 65536), (2000, 257 + 1800)],
+    "batch_pairs": [(3, 16384), (4, 16385), (2999, 24576)],
+}
+
+
+def _matrix(name, n=70001, seed=5):
+    rng = np.random.default_rng(seed)
+    lengths = rng.integers(0, 41, 3001)
+    lengths[rng.integers(0, 3001, 60)] = 0
+    for at, length in LONG[name]:
+        lengths[at] = length
+    rp, col = csr_from_lengths([int(v) for v in lengths], n, rng)
+    return rp, col, n
+
+
+@pytest.fixture(autouse=True)
+def split_rows_table(tmp_path):
+    """Table rows as the shipped table has at these sizes: split-row tiles, or row groups beside long rows."""
+    t = tmp_path / "table.txt"
+    t.write_text("".join(f"t -1 {rows} {d} flat {tile} 0 0 0 0\n" for d in ("f64", "f32", "f16")
+                         for rows in ("dense", "skewed") for tile in (16, 2048)))
+    pf.set_tuning_table(str(t))
+    yield
+    pf.set_tuning_table(None)
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_long_rows_beside_row_groups(name, dtype):
+    rp, col, n = _matrix(name)
+    kv, kx = oracle.initvec(len(col), NP[dtype]), oracle.initvec(n, NP[dtype])
+    y, info = gpu_spmv(rp, col, kv, kx, "auto", dtype=dtype)
+    assert (info["variant_name"], info["tile"], info["hybrid"]) == ("flat", 16, 0), info
+    assert_parity(rp, col, kv, kx, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{name}/kat")
+    rng = np.random.default_rng(1)
+    val = rng.uniform(-1, 1, len(col)).astype(NP[dtype])
+    x = rng.uniform(-1, 1, n).astype(NP[dtype])
+    y, _ = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
+    assert_parity(rp, col, val, x, y, dtype, what=f"{name}/random")
+
+
+@pytest.mark.parametrize("what,change", [
+    ("a row over 2^16", lambda l: l.__setitem__(5, 65537)),
+    ("a short row over 128", lambda l: l.__setitem__(5, 129)),
+    ("long rows under 1024 on average", lambda l: l.__setitem__(1500, 900)),
+    ("short rows under 12 on average", lambda l: l.__setitem__(slice(2000, None), 0)),
+])
+def test_rule_refuses(what, change):
+    rng = np.random.default_rng(6)
+    lengths = rng.integers(4, 24, 3001)
+    lengths[1500] = 3000
+    change(lengths)
+    rp, col = csr_from_lengths([int(v) for v in lengths], 70001, rng)
+    val, x = oracle.initvec(len(col)), oracle.initvec(70001)
+    y, info = gpu_spmv(rp, col, val, x, "auto")
+    assert info["tile"] == 2048, (what, info)
+    assert_parity(rp, col, val, x, y, "f64", exact=True, what=what)
+
+
+def test_special_values_and_graph_replay():
+    rp, col, n = _matrix("adjacent")
+    rng = np.random.default_rng(2)
+    val, x = oracle.initvec(len(col)), oracle.initvec(n)
+    for a in (val, x):
+        at = rng.choice(len(a), 40, replace=False)
+        a[at] = np.resize([np.nan, np.inf, -np.inf], 40)
+    want = oracle.spmv_serial(rp, col, val, x)
+    d = [dev(a) for a in (rp, col, val, x)]
+    y = torch.full((len(rp) - 1,), 7.0, dtype=torch.float64, device=DEV)
+    with pf.Plan(d[0], d[1], len(rp) - 1, n, len(col)) as p:
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            p.execute(*d, y, stream=s)
+            s.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                p.execute(*d, y, stream=s)
+        for _ in range(3):
+            y.fill_(7.0)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
+            d[2].mul_(1.0)  # eager work between the replays
+        p.check()
+
+
+def test_row_ptr_changed_after_planning_is_flagged():
+    rp, col, n = _matrix("one")
+    val, x = oracle.initvec(len(col)), oracle.initvec(n)
+    d = [dev(a) for a in (rp, col, val, x)]
+    y = torch.empty(len(rp) - 1, dtype=torch.float64, device=DEV)
+    other = rp.copy()
+    other[1501:] -= 2900  # the listed row now holds 100 nnz (in bounds throughout)
+    with pf.Plan(d[0], d[1], len(rp) - 1, n, len(col)) as p:
+        assert p.info.tile == 16
+        p.execute(dev(other), d[1], d[2], d[3], y)
+        with pytest.raises(pf.PrefreeError) as e:
+            p.check()
+        assert pf.STATUS[e.value.status] == "PF_ERR_KERNEL"
