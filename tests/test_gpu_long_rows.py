@@ -106,16 +106,21 @@ def test_special_values_and_graph_replay():
         p.check()
 
 
-def test_row_ptr_changed_after_planning_is_flagged():
+@pytest.mark.parametrize("what", ["a listed row now short", "another row now long"])
+def test_row_ptr_changed_after_planning_is_flagged(what):
     rp, col, n = _matrix("one")
     val, x = oracle.initvec(len(col)), oracle.initvec(n)
     d = [dev(a) for a in (rp, col, val, x)]
-    y = torch.empty(len(rp) - 1, dtype=torch.float64, device=DEV)
-    other = rp.copy()
-    other[1501:] -= 2900  # the listed row now holds 100 nnz (in bounds throughout)
+    y = torch.full((len(rp) - 1,), float("nan"), dtype=torch.float64, device=DEV)
+    other = rp.copy()  # in bounds throughout
+    if what == "a listed row now short":
+        other[1501:] -= 2900
+    else:
+        other[1498:1501] = other[1500] + 1000  # row 1497 takes over the rows to 1499 and 1000 nnz of the listed row
     with pf.Plan(d[0], d[1], len(rp) - 1, n, len(col)) as p:
         assert p.info.tile == 16
         p.execute(dev(other), d[1], d[2], d[3], y)
+        assert np.array_equal(y.cpu().numpy(), oracle.spmv_serial(other, col, val, x))  # and every row summed
         with pytest.raises(pf.PrefreeError) as e:
             p.check()
         assert pf.STATUS[e.value.status] == "PF_ERR_KERNEL"
