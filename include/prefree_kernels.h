@@ -142,8 +142,9 @@ typedef struct pfk_spmv_args {
 /* nnz per long-row tile of a hybrid plan in long mode. */
 #define PFK_LONG_TILE 1024
 
-/* Row groups beside long rows (pfk_spmv_flat, tile = PFK_VECTOR_LONG_LANES, n_dense > 0): dense_rows lists the rows
- * over PFK_ALIGN_ROW_MAX nnz, each once; a workgroup sums each of them whole and the row groups the others. */
+/* Row groups beside long rows (pfk_spmv_flat, tile = PFK_VECTOR_LONG_LANES, n_dense > 0): dense_rows lists the n_dense
+ * rows over PFK_ALIGN_ROW_MAX nnz, each once, and holds a bitmap of them behind the list, bit r & 31 of word r >> 5 for
+ * row r, (m + 31) / 32 words; a workgroup sums each of them whole and the row groups the others. */
 #define PFK_VECTOR_LONG_LANES 16
 
 /* Bytes of one split-row partial (head / tail slot): fp32 in the fp16 mode. */

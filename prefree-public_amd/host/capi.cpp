@@ -1002,19 +1002,23 @@ bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanS
 }
 
 // The list of a row-groups-beside-long-rows plan on the device, longest row first (the long rows start with the
-// call).  Synchronises `stream`.
+// call), and behind it a bitmap of the same rows (see PFK_VECTOR_LONG_LANES).  Synchronises `stream`.
 int add_long_rows(pf_plan *p, const PlanScan &scan, void *stream)
 {
     const size_t count = (size_t)scan.host_n;
-    std::vector<int> order(count), rows(count);
+    std::vector<int> order(count), rows(count + ((size_t)p->m + 31) / 32, 0);
     for (size_t k = 0; k < count; ++k) order[k] = (int)k;
     const auto len = [&](int k) { return scan.host[(size_t)(4 * k + 2)] - scan.host[(size_t)(4 * k + 1)]; };
     std::sort(order.begin(), order.end(), [&](int x, int y) {
         return len(x) != len(y) ? len(x) > len(y) : scan.host[(size_t)(4 * x)] < scan.host[(size_t)(4 * y)];
     });
-    for (size_t k = 0; k < count; ++k) rows[k] = scan.host[(size_t)(4 * order[k])];
-    PF_TRY(pfk_malloc(reinterpret_cast<void **>(&p->long_rows), count * sizeof(int)), "long-row list");
-    int st = pfk_memcpy_h2d(p->long_rows, rows.data(), count * sizeof(int), stream);
+    for (size_t k = 0; k < count; ++k) {
+        const int r = scan.host[(size_t)(4 * order[k])];
+        rows[k] = r;
+        rows[count + (size_t)(r >> 5)] |= (int)(1u << (r & 31));
+    }
+    PF_TRY(pfk_malloc(reinterpret_cast<void **>(&p->long_rows), rows.size() * sizeof(int)), "long-row list");
+    int st = pfk_memcpy_h2d(p->long_rows, rows.data(), rows.size() * sizeof(int), stream);
     if (st == PF_OK) st = pfk_stream_sync(stream);
     if (st != PF_OK) return from_kernel_layer(st, "long-row list");
     p->n_long_rows = (int)count;
