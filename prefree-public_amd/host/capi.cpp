@@ -57,6 +57,7 @@ constexpr long long kRowGroupBytesMax = 256LL << 20;
 constexpr long long kRowGroupWideBytesMax = 64LL << 20;  // over 2^18 rows (see auto_choice)
 constexpr long long kVectorLongBytesMax = 128LL << 20;  // see vector_long_rule
 constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
+constexpr int kBandDefaultMin = 4096;  // see try_band
 
 // Tiles per XCD list of an x-window schedule: an even share plus 2% slack.
 long long sched_cap(long long ntiles) { return (ntiles + kXcds - 1) / kXcds + ntiles / 400 + 1; }
@@ -78,9 +79,18 @@ int value_bytes(int dtype) { return dtype == PF_F64 ? 8 : dtype == PF_F32 ? 4 : 
 // 32.6 instead of 33.7 in fp16, and C3 (split rows) 213.8 instead of 216.3.
 // Matrices of very short rows (under 4 nnz on average, as C4: 2.5) keep one
 // chunk per XCD: their x neighbourhood spans more rows than a chunk holds, and
-// chunks of 2^15 nnz cost 1-2 us of 320 there (2^12: 354 us).
+// chunks of 2^15 nnz cost 1-2 us of 320 there (2^12: 354 us).  Matrices of up to
+// 4M nnz with long rows take 2^13: 2^15 leaves an XCD about ten chunks, whose
+// rows differ too much to even out (power law, 1024-nnz tiles, us per call at
+// 2^13 and 2^15: 1.35M nnz fp64 14.8 and 15.1, fp32 13.2 and 13.4; 3.7M nnz fp64
+// 28.8 and 29.9, fp16 20.6 and 21.7; 4.6M nnz fp64 40.4 and 40.0, 7.6M equal).
 constexpr long long kChunkNnz = 1LL << 15;
-long long chunk_rule(const pf_row_stats &s) { return s.nnz < 4LL * s.m ? 0 : kChunkNnz; }
+constexpr long long kChunkSkewNnz = 1LL << 13;
+long long chunk_rule(const pf_row_stats &s)
+{
+    if (s.nnz < 4LL * s.m) return 0;
+    return s.max_row_len > PFK_ALIGN_ROW_MAX && s.nnz < 4000000 ? kChunkSkewNnz : kChunkNnz;
+}
 // Bytes of one split-row partial sum (head / tail slot): fp32 in the fp16 mode.
 int slot_bytes(int dtype) { return dtype == PF_F16 ? 4 : value_bytes(dtype); }
 
@@ -1030,7 +1040,10 @@ int add_long_rows(pf_plan *p, const PlanScan &scan, void *stream)
 // smallest w that holds 85% of the nnz and, with two steps' rows, fits the
 // kernel's LDS ring.  On by
 // default for matrices of under 4 nnz per row on average (each row's x entry
-// is then a large part of the stream, and the band's gathers cost most).
+// is then a large part of the stream, and the band's gathers cost most) whose
+// band is wide: within a narrow one the tiles' gathers share lines (8M rows of 3
+// columns within +-w, band against 2048-nnz tiles, us per call: w 100 fp64 106.7
+// and 68.4, fp32 68.6 and 46.3; w 1500 fp64 108.0 and 80.8, fp32 69.4 and 53.3).
 int try_band(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream, PlanTimer *timer)
 {
     const pf_plan_info &in = p->info;
@@ -1058,7 +1071,7 @@ int try_band(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream, P
             break;
         }
     }
-    p->info.band_w = (p->band_avail > 0 && nnz < 4 * m) ? p->band_avail : 0;
+    p->info.band_w = (p->band_avail >= kBandDefaultMin && nnz < 4 * m) ? p->band_avail : 0;
     return PF_OK;
 }
 
@@ -1155,6 +1168,7 @@ int check_matrix_args(const int *d_row_ptr, const int *d_col, int m, int n, int 
     if (m > 0 && !d_row_ptr) return fail(PF_ERR_INVALID, "row_ptr is NULL");
     if ((unsigned long long)nnz + (unsigned long long)m >= 0xFFFFFFFFull)
         return fail(PF_ERR_UNSUPPORTED, "nnz + m must stay below 2^32");
+    if (rc == PF_OK && !allow_hybrid) p->info.band_w = 0;  // a table row of plain tiles (pf_plan_set_band brings it back)
     // x and y are addressed through buffer resources with 32-bit byte offsets.
     if ((unsigned long long)n * (unsigned long long)value_bytes(dtype) >= 0xFFFFFFF0ull ||
         (unsigned long long)m * (unsigned long long)value_bytes(dtype) >= 0xFFFFFFF0ull)

@@ -123,6 +123,42 @@ def test_band_default_rule():
     torch.cuda.synchronize()
 
 
+def test_band_default_needs_a_wide_band():
+    """Columns within +-1000 of their rows: the plan finds the band (to be switched on) and keeps its tiles."""
+    rp, col = _banded(700000, 3.0, 1000, 0.0, seed=6)[:2]
+    n = len(rp) - 1
+    with pf.Plan(dev(rp), dev(col), n, n, len(col), "f64", "auto") as p:
+        assert p.info.band_w == 0
+        p.set_band(True)
+        assert 0 < p.info.band_w < 4096
+    torch.cuda.synchronize()
+
+
+def test_table_row_of_plain_tiles(tmp_path):
+    """A table row with hybrid 0 keeps a banded plan's tiles; pf_plan_set_band switches the band on, same y."""
+    name, rp, col, n = CASES[0]
+    m = len(rp) - 1
+    val, x = oracle.initvec(len(col)), oracle.initvec(n)
+    d = [dev(a) for a in (rp, col, val, x)]
+    y = torch.full((m,), float("nan"), dtype=torch.float64, device="cuda:0")
+    for hybrid, band in ((0, 0), (1, 4096)):
+        t = tmp_path / f"table{hybrid}.txt"
+        t.write_text(f"t -1 short f64 flat 2048 0 0 0 {hybrid}\n")
+        pf.set_tuning_table(str(t))
+        try:
+            p = pf.Plan(d[0], d[1], m, n, len(col), "f64", "auto")
+        finally:
+            pf.set_tuning_table(None)
+        with p:
+            assert (p.info.tile, p.info.band_w) == (2048, band)
+            for on in (False, True):
+                if on:
+                    p.set_band(True)
+                for _ in range(2):  # the first call records the map
+                    p.execute(*d, y)
+                    assert_parity(rp, col, val, x, y.cpu().numpy(), "f64", exact=True, what=f"{name} {hybrid} {on}")
+
+
 def test_band_plan_searching_every_call():
     """A band plan told to search its rows on every call (pf_plan_set_remember_rows(plan, 0)) searches its row
     map afresh before each band kernel, with the remembering plan's y; switching back records the map again."""
