@@ -2394,6 +2394,44 @@ __global__ __launch_bounds__(kBandBS) void k_band(Args<T> a, BandArgs b)
 // global atomics per workgroup (at most kBandStatsWg workgroups).
 constexpr int kBandStatsWg = 512;
 
+// How far neighbouring rows' columns lie apart: over kScatterRows rows spread
+// over the matrix, at most 16 entries each, out[0] = the entries whose column
+// lies within PFK_SCATTER_NEAR of the next row's entry of the same position,
+// out[1] = the entries compared.  A stencil or a band has nearly all of them
+// near, whatever block of rows of it this is; random columns few.  One
+// workgroup: some microseconds, once per plan that asks.
+constexpr int kScatterBS = 1024;
+constexpr int kScatterRows = 2 * kScatterBS;
+
+__global__ __launch_bounds__(kScatterBS) void k_scatter_stats(const int *__restrict__ rp, const int *__restrict__ col,
+                                                              int m, int nnz, unsigned int *__restrict__ out)
+{
+    __shared__ unsigned int s_n[2];
+    const int tid = threadIdx.x;
+    if (tid < 2) s_n[tid] = 0;
+    __syncthreads();
+    unsigned int near = 0, all = 0;
+    for (int i = tid; i < kScatterRows; i += kScatterBS) {
+        const long long r = (long long)(m - 1) * i / kScatterRows;  // r + 1 < m, where m > 1
+        if (r + 1 >= m) break;
+        const int a = min(max(rp[r], 0), nnz), b = min(max(rp[r + 1], a), nnz), c = min(max(rp[r + 2], b), nnz);
+        const int len = min(min(b - a, c - b), 16);
+        for (int k = 0; k < len; ++k) {
+            near += llabs((long long)col[a + k] - col[b + k]) <= PFK_SCATTER_NEAR ? 1u : 0u;
+            ++all;
+        }
+    }
+    const auto add = [](unsigned int x, unsigned int y) { return x + y; };
+    near = wave_reduce_u32(near, add);
+    all = wave_reduce_u32(all, add);
+    if ((tid & (kWave - 1)) == 0) {
+        atomicAdd(&s_n[0], near);
+        atomicAdd(&s_n[1], all);
+    }
+    __syncthreads();
+    if (tid < 2) out[tid] = s_n[tid];
+}
+
 __global__ __launch_bounds__(kBS) void k_band_stats(const int *__restrict__ rp, const int *__restrict__ col, int m,
                                                     unsigned long long *__restrict__ out)
 {
@@ -5071,6 +5109,14 @@ int pfk_band_stats(const int *row_ptr, const int *col, int m, unsigned long long
                            S(stream), row_ptr, col, m, out);
         PFK_LAUNCHED("k_band_stats");
     }
+    return PF_OK;
+}
+
+int pfk_scatter_stats(const int *row_ptr, const int *col, int m, int nnz, unsigned int *out, void *stream)
+{
+    if (!row_ptr || !out || m < 0 || nnz < 0 || (nnz > 0 && !col)) return PF_ERR_INVALID;
+    hipLaunchKernelGGL(k_scatter_stats, dim3(1), dim3(kScatterBS), 0, S(stream), row_ptr, col, m, nnz, out);
+    PFK_LAUNCHED("k_scatter_stats");
     return PF_OK;
 }
 

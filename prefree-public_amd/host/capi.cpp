@@ -55,6 +55,7 @@ constexpr long long kXcdL2Bytes = 4LL << 20;  // MI355X: 4 MB of L2 per XCD
 constexpr long long kRowGroupRowsMax = 1LL << 18;
 constexpr long long kRowGroupBytesMax = 256LL << 20;
 constexpr long long kRowGroupWideBytesMax = 64LL << 20;  // over 2^18 rows (see auto_choice)
+constexpr long long kRowGroupWide12BytesMax = 88LL << 20;  // the same for 12 or more nnz per row
 constexpr long long kVectorLongBytesMax = 128LL << 20;  // see vector_long_rule
 constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
 constexpr int kBandDefaultMin = 4096;  // see try_band
@@ -280,6 +281,7 @@ struct Choice {
     int variant = PF_ADAPTIVE, tile = 0, run = 0, keep = -1, ladder = 0;
     bool hybrid = true;
     bool beside = true;  // row groups beside long rows, where vector_long_rule takes them
+    int scattered = 0;   // lanes per row of the row groups that a plan whose columns are scattered takes (0: none)
 };
 
 bool table_choice(const pf_row_stats &s, int dtype, Choice &c)
@@ -338,14 +340,19 @@ int row_group_lanes(const pf_row_stats &s)
 //     tiles; 131072 rows of 32 nnz 24.8 against 28.7; 262144 x 64 86 against
 //     99; 262144 x 128, 403 MB, 239 against 192 for 2048-nnz tiles);
 //   * more rows, none longer than 64, of 7 to 16 nnz on average, values and
-//     columns within 64 MB: row groups too.  A tile's barriers and LDS round
-//     trip hold its gathers back where a call is little more than one round of
-//     tiles; 300007 rows of 16 random columns, fp64 34.3 us for 1024-nnz tiles,
-//     28.6 for 8 lanes per row, fp32 29.0 and 24.7, fp16 25.8 and 23.1; rows of
-//     8: 20.7 and 16.4 (fp64).  The lines: 16-nnz rows over 115 MB (600000,
-//     fp64) take 82 us against 71 for tiles, 77 MB (fp32) 48.4 against 51.3;
-//     24-nnz rows 49.7 against 48.3 and 27-point stencils 31.3 against 27.4
-//     (300000, fp64); 5-point grids take tiles at every size over 2^18 rows;
+//     columns within 64 MB, or 88 MiB for 12 nnz per row and more: row groups
+//     too in a plan that finds the columns scattered (scattered_columns), where
+//     every gather is a line of its own whoever makes it and a tile's barriers
+//     and LDS round trip hold the gathers back.  Where rows follow each other's
+//     columns the tiles' gathers share lines and row groups lose: 9-point
+//     stencils, 560000 rows, fp64 13.6 us for tiles, 20.6 for row groups, fp32
+//     10.9 and 15.5, fp16 10.0 and 13.2.  300007 rows of 16 random columns: fp64
+//     32.0 us for 1024-nnz tiles, 26.3 for 16 lanes per row (27.7 for 8), fp32
+//     27.1, 23.9 and 24.2, fp16 24.6, 23.1 and 22.3; rows of 8: 20.7 and 16.4
+//     (fp64).  The lines: 16-nnz rows over 86 MB (450000, fp64) take 44.7 us with
+//     16 lanes against 47.2 for tiles, 90 MB (700000, fp32) 53.6 against 56.7,
+//     102 MB (800000, fp32) 66.0 against 64.1, 115 MB (600000, fp64) 68.0 against
+//     69.0, 134 MB (700000, fp64) 92 against 84; 24-nnz rows 49.7 against 48.3;
 //   * no row longer than PFK_ALIGN_ROW_MAX, or fp16 values (FLAT only): FLAT
 //     (1024 nnz per tile for fp64, 2048 for fp32 / fp16 or for rows of under
 //     4 nnz on average), row-aligned when the rows fit: one launch per call;
@@ -368,11 +375,14 @@ Choice auto_choice(const pf_row_stats &s, int dtype)
     c.variant = PF_FLAT;
     const long long stream = nnz * (value_bytes(dtype) + 4);
     const bool few = m <= kRowGroupRowsMax && stream <= kRowGroupBytesMax;
-    const bool middling = s.max_row_len <= 64 && nnz >= 7 * m && nnz <= 16 * m + m / 2 && stream <= kRowGroupWideBytesMax;
-    if (s.max_row_len <= PFK_ALIGN_ROW_MAX && m > 0 && (few || middling)) {
+    if (s.max_row_len <= PFK_ALIGN_ROW_MAX && m > 0 && few) {
         c.tile = row_group_lanes(s);
         return c;
     }
+    const bool twelve = nnz >= 12 * m;
+    if (s.max_row_len <= 64 && nnz >= 7 * m && nnz <= 16 * m + m / 2 &&
+        stream <= (twelve ? kRowGroupWide12BytesMax : kRowGroupWideBytesMax))
+        c.scattered = twelve && dtype != PF_F16 ? 16 : row_group_lanes(s);
     if (s.max_row_len <= PFK_ALIGN_ROW_MAX || dtype == PF_F16) {
         c.tile = default_tile(PF_FLAT, dtype);
         // Rows of under 4 nnz on average: a tile spends much of its time per
@@ -574,7 +584,7 @@ namespace {
 // hybrid: always, unless a tuning-table row says otherwise; `allow_beside`
 // whether row groups beside long rows may replace it.
 int plan_info(const pf_row_stats &s, int n, int dtype, int variant, int tile, pf_plan_info *out,
-              bool *allow_hybrid = nullptr, bool *allow_beside = nullptr)
+              bool *allow_hybrid = nullptr, bool *allow_beside = nullptr, int *scattered = nullptr)
 {
     Choice c;
     if (allow_hybrid) *allow_hybrid = true;
@@ -583,6 +593,7 @@ int plan_info(const pf_row_stats &s, int n, int dtype, int variant, int tile, pf
         c = auto_choice(s, dtype);
         if (allow_hybrid) *allow_hybrid = c.hybrid;
         if (allow_beside) *allow_beside = c.beside;
+        if (scattered) *scattered = c.scattered;
         variant = c.variant;
         if (tile <= 0 || !tile_supported(variant, dtype, tile)) tile = c.tile;
     }
@@ -1075,6 +1086,24 @@ int try_band(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream, P
     return PF_OK;
 }
 
+// Whether fewer than a quarter of the sampled entries lie within PFK_SCATTER_NEAR columns of the next row's (random
+// columns over 300,000: 2%; stencils and bands: nearly all of them).  Synchronises `stream`.
+int scattered_columns(const int *d_row_ptr, const int *d_col, int m, int nnz, void *stream, PlanTimer *timer, bool *yes)
+{
+    unsigned int *d = nullptr;
+    unsigned int h[2] = {0, 0};
+    PF_TRY(pfk_malloc(reinterpret_cast<void **>(&d), sizeof h), "column statistic");
+    if (timer) timer->start(stream);
+    int st = pfk_scatter_stats(d_row_ptr, d_col, m, nnz, d, stream);
+    if (st == PF_OK) st = pfk_memcpy_d2h(h, d, sizeof h, stream);
+    if (st == PF_OK) st = pfk_stream_sync(stream);
+    if (st == PF_OK && timer) timer->stop(stream);
+    pfk_free(d);
+    if (st != PF_OK) return from_kernel_layer(st, "column statistic");
+    *yes = 4ull * h[0] < h[1];
+    return PF_OK;
+}
+
 // The plan for a validated matrix with known statistics (shared by plan
 // creation and the tuner's candidates): workspace allocated and initialised.
 // With columns given, PF_AUTO and PF_FLAT plans of the default tile also try
@@ -1085,7 +1114,8 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
 {
     bool allow_hybrid = true, allow_beside = false;
     pf_plan_info info;
-    const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid, &allow_beside);
+    int scattered = 0;
+    const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid, &allow_beside, &scattered);
     bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && allow_hybrid;
     if (st != PF_OK) return st;
     bool beside = false;  // row groups beside long rows
@@ -1095,6 +1125,12 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         if (st2 != PF_OK) return st2;
         beside = true;
         want_hybrid = false;
+    }
+    if (scattered > 0 && tile <= 0 && d_col) {
+        bool yes = false;
+        int st2 = scattered_columns(d_row_ptr, d_col, m, nnz, stream, timer, &yes);
+        if (st2 == PF_OK && yes) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
+        if (st2 != PF_OK) return st2;
     }
     pf_plan *p = new pf_plan();
     p->m = m;

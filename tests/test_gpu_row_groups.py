@@ -118,3 +118,29 @@ def test_auto_over_2_18_rows_of_middling_length(extra, longest, groups, dtype):
     y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
     assert (info["variant_name"], info["tile"] <= 32) == ("flat", groups), info
     assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{extra} {longest} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("block", [1, 2])
+@pytest.mark.parametrize("pattern,groups", [("9-point", False), ("random", True)])
+def test_auto_over_2_18_rows_looks_at_the_columns(pattern, groups, block, dtype):
+    """9 columns a row: a stencil keeps its tiles, whole or as the second half of its rows (whose columns lie far from
+    its local row numbers); random columns take row groups."""
+    side = 513 if block == 1 else 726
+    n = side * side
+    if pattern == "random":
+        rng = np.random.default_rng(8)
+        cols = np.sort(rng.integers(0, n, (n, 9)), axis=1)
+    else:
+        d = np.array([-1, 0, 1])
+        cols = np.arange(n)[:, None] + (side * d[:, None] + d[None, :]).ravel()[None, :]
+    cols = cols[n - n // block:]
+    ok = (cols >= 0) & (cols < n)
+    rp = np.zeros(len(cols) + 1, dtype=np.int32)
+    rp[1:] = np.cumsum(ok.sum(1))
+    col = cols[ok].astype(np.int32)
+    assert len(cols) > 1 << 18
+    val, x = oracle.initvec(len(col), NP[dtype]), oracle.initvec(n, NP[dtype])
+    y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
+    assert (info["variant_name"], info["tile"] <= 32) == ("flat", groups), info
+    assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{pattern} {block} {dtype}")
