@@ -3418,10 +3418,12 @@ __global__ __launch_bounds__(kBS) void k_vector(Args<T> a)
 constexpr int kVecBS = 1024;
 constexpr int kVecU = 8;
 
+// fp64 takes 71 registers, one workgroup per CU; batches of 4 (57, two per CU) lose: 20,011 rows 8.0 -> 8.9 us.
 template <typename T, int L>
 __global__ __launch_bounds__(kVecBS) void k_vector_long(Args<T> a, const int *__restrict__ rows, int nlong)
 {
     using P = acc_t<T>;
+    constexpr int U = kVecU;
     __shared__ P s_red[kVecBS / kWave];
     const int tid = threadIdx.x;
     const int nnz = a.nnz;
@@ -3456,12 +3458,10 @@ __global__ __launch_bounds__(kVecBS) void k_vector_long(Args<T> a, const int *__
             P p[U];  // a batch's products as a tree, then to the lane's sum: few roundings in a row where 60 were
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-// fp64 takes 71 registers, one workgroup per CU; batches of 4 (57, two per CU) lose: 20,011 rows 8.0 -> 8.9 us.
                 const int q = b + u * kVecBS + tid;
                 p[u] = q >= lead && q < len ? P(v[u]) * P(xv[u]) : P(0);
             }
 #pragma unroll
-    constexpr int U = kVecU;
             for (int h = U / 2; h > 0; h /= 2)
 #pragma unroll
                 for (int u = 0; u < h; ++u) p[u] += p[u + h];
@@ -3486,6 +3486,9 @@ __global__ __launch_bounds__(kVecBS) void k_vector_long(Args<T> a, const int *__
     const int q = tid & (L - 1);
     if (g >= a.m)
         return;  // whole groups
+    // The row's bit in the list's bitmap, read beside row_ptr: looking a long row up in the list itself put one
+    // more latency on its wave (120,011 rows fp32 30.4 us, 30.2 with the bitmap, 29.9 unchecked).
+    const bool listed = ((unsigned)rows[nlong + (g >> 5)] >> (g & 31)) & 1u;
     const int r0 = min(max(a.rp[g], 0), nnz);
     const int r1 = min(max(a.rp[g + 1], r0), nnz);
     bool apart = r1 - r0 > kAlignRowMax;
@@ -3519,9 +3522,6 @@ __device__ __forceinline__ T half_wave_tree(T v)
 }
 
 template <typename T>
-    // The row's bit in the list's bitmap, read beside row_ptr: looking a long row up in the list itself put one
-    // more latency on its wave (120,011 rows fp32 30.4 us, 30.2 with the bitmap, 29.9 unchecked).
-    const bool listed = ((unsigned)rows[nlong + (g >> 5)] >> (g & 31)) & 1u;
 __device__ __forceinline__ void atomic_add(T *p, T v) { atomicAdd(p, v); }
 
 // Sum over the aligned groups of V lanes of each 32-lane half, as lane 0 of a

@@ -57,8 +57,8 @@ constexpr long long kRowGroupBytesMax = 256LL << 20;
 constexpr long long kRowGroupWideBytesMax = 64LL << 20;  // over 2^18 rows (see auto_choice)
 constexpr long long kRowGroupWide12BytesMax = 88LL << 20;  // the same for 12 or more nnz per row
 constexpr long long kVectorLongBytesMax = 128LL << 20;  // see vector_long_rule
-constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
 constexpr int kBandDefaultMin = 4096;  // see try_band
+constexpr long long kChipLanes = 256LL * 2048;  // lanes resident on the chip: 256 CUs x 32 waves x 64
 
 // Tiles per XCD list of an x-window schedule: an even share plus 2% slack.
 long long sched_cap(long long ntiles) { return (ntiles + kXcds - 1) / kXcds + ntiles / 400 + 1; }
@@ -1168,6 +1168,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         }
     }
     if (rc == PF_OK && d_col && !candidate) rc = try_band(p, d_row_ptr, d_col, stream, timer);
+    if (rc == PF_OK && !allow_hybrid) p->info.band_w = 0;  // a table row of plain tiles (pf_plan_set_band brings it back)
     if (rc == PF_OK && candidate) {
         rc = try_hybrid(p, d_row_ptr, d_col, stream, scan, timer);
         if (rc == PF_OK && !p->hybrid) {  // stays split-row: its workspace now
@@ -1204,7 +1205,6 @@ int check_matrix_args(const int *d_row_ptr, const int *d_col, int m, int n, int 
     if (m > 0 && !d_row_ptr) return fail(PF_ERR_INVALID, "row_ptr is NULL");
     if ((unsigned long long)nnz + (unsigned long long)m >= 0xFFFFFFFFull)
         return fail(PF_ERR_UNSUPPORTED, "nnz + m must stay below 2^32");
-    if (rc == PF_OK && !allow_hybrid) p->info.band_w = 0;  // a table row of plain tiles (pf_plan_set_band brings it back)
     // x and y are addressed through buffer resources with 32-bit byte offsets.
     if ((unsigned long long)n * (unsigned long long)value_bytes(dtype) >= 0xFFFFFFF0ull ||
         (unsigned long long)m * (unsigned long long)value_bytes(dtype) >= 0xFFFFFFF0ull)
