@@ -2395,13 +2395,14 @@ __global__ __launch_bounds__(kBandBS) void k_band(Args<T> a, BandArgs b)
 constexpr int kBandStatsWg = 512;
 
 // How far neighbouring rows' columns lie apart: over kScatterRows rows spread
-// over the matrix, at most 16 entries each, out[0] = the entries whose column
+// over the matrix, their first kScatterPer entries, out[0] = the entries whose column
 // lies within PFK_SCATTER_NEAR of the next row's entry of the same position,
 // out[1] = the entries compared.  A stencil or a band has nearly all of them
 // near, whatever block of rows of it this is; random columns few.  One
-// workgroup: some microseconds, once per plan that asks.
+// workgroup, 7.7 us once per plan that asks (a lane per row, 2048 rows: 41.4).
 constexpr int kScatterBS = 1024;
-constexpr int kScatterRows = 2 * kScatterBS;
+constexpr int kScatterRows = 256;
+constexpr int kScatterPer = 16;  // entries of a row, a lane each: two latencies a pass, four passes in flight
 
 __global__ __launch_bounds__(kScatterBS) void k_scatter_stats(const int *__restrict__ rp, const int *__restrict__ col,
                                                               int m, int nnz, unsigned int *__restrict__ out)
@@ -2411,15 +2412,15 @@ __global__ __launch_bounds__(kScatterBS) void k_scatter_stats(const int *__restr
     if (tid < 2) s_n[tid] = 0;
     __syncthreads();
     unsigned int near = 0, all = 0;
-    for (int i = tid; i < kScatterRows; i += kScatterBS) {
-        const long long r = (long long)(m - 1) * i / kScatterRows;  // r + 1 < m, where m > 1
-        if (r + 1 >= m) break;
+    const int k = tid % kScatterPer;
+#pragma unroll
+    for (int i0 = 0; i0 < kScatterRows; i0 += kScatterBS / kScatterPer) {
+        const long long r = (long long)(m - 1) * (i0 + tid / kScatterPer) / kScatterRows;  // r + 1 < m, where m > 1
+        if (r + 1 >= m) continue;
         const int a = min(max(rp[r], 0), nnz), b = min(max(rp[r + 1], a), nnz), c = min(max(rp[r + 2], b), nnz);
-        const int len = min(min(b - a, c - b), 16);
-        for (int k = 0; k < len; ++k) {
-            near += llabs((long long)col[a + k] - col[b + k]) <= PFK_SCATTER_NEAR ? 1u : 0u;
-            ++all;
-        }
+        if (k >= min(b - a, c - b)) continue;
+        near += llabs((long long)col[a + k] - col[b + k]) <= PFK_SCATTER_NEAR ? 1u : 0u;
+        ++all;
     }
     const auto add = [](unsigned int x, unsigned int y) { return x + y; };
     near = wave_reduce_u32(near, add);
