@@ -263,7 +263,10 @@ int pf_set_tuning_table(const char *path);
 /* Path of the table PF_AUTO consults ("" when none). */
 const char *pf_tuning_table(void);
 
-/* One-shot y = A·x: plan, execute, synchronise, destroy. */
+/* One-shot y = A·x: plan, execute, synchronise, destroy.  PF_AUTO with up to 2^26 nnz chooses by the row statistics
+ * alone (as pf_spmv_noalloc does; no hybrid plan, no row groups found from the long rows or the columns) and works in
+ * pf_spmv_noalloc's scratch array, or, while another call is in it, in an allocation of its own: y is the same either
+ * way, bit for bit.  It may differ in its last bits from the y of a plan made by pf_plan_create. */
 int pf_spmv(const int *d_row_ptr, const int *d_col, const void *d_val, const void *d_x, void *d_y,
             int m, int n, int nnz, int dtype, int variant, void *stream);
 
@@ -277,7 +280,8 @@ int pf_spmv(const int *d_row_ptr, const int *d_col, const void *d_val, const voi
  * called on a stream that is capturing a HIP graph: a caller who captures makes a plan before the capture
  * (pf_plan_create) and captures pf_plan_execute.  Calls on one device from several host threads are
  * serialised by a per-device lock in this library, since they share the one array; each call has
- * finished with it when it returns. */
+ * finished with it when it returns.  A pf_spmv call that is in the array (see there) holds the same lock
+ * until its stream has drained. */
 int pf_spmv_noalloc(const int *d_row_ptr, const int *d_col, const void *d_val, const void *d_x, void *d_y,
                     int m, int n, int nnz, int dtype, int variant, void *stream);
 

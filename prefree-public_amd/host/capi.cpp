@@ -1707,8 +1707,8 @@ int pf_plan_destroy(pf_plan *plan)
     return st == PF_OK ? PF_OK : from_kernel_layer(st, "free workspace");
 }
 
-// One-shot y = A x with its statistics and workspace in the device's scratch array, under the lock the caller holds
-// (`scratch_lock`), until the stream is synchronised.
+// One-shot y = A x with its statistics and workspace in `scr`, the caller's until this returns: the device's scratch
+// array under its lock, or an allocation of the same size.  The stream has drained on return, whatever the status.
 static int spmv_in_scratch(void *scr, size_t scr_bytes, const int *d_row_ptr, const int *d_col, const void *d_val,
                            const void *d_x, void *d_y, int m, int n, int nnz, int dtype, int variant, void *stream)
 {
@@ -1717,7 +1717,10 @@ static int spmv_in_scratch(void *scr, size_t scr_bytes, const int *d_row_ptr, co
     p.n = n;
     p.nnz = nnz;
     int st = stats_via(static_cast<unsigned long long *>(scr), d_row_ptr, d_col, m, n, nnz, &p.stats, stream);
-    if (st != PF_OK) return st;
+    if (st != PF_OK) {
+        pfk_stream_sync(stream);
+        return st;
+    }
     st = check_csr_stats(p.stats, nnz);
     if (st != PF_OK) return st;
     st = plan_info(p.stats, n, dtype, variant, 0, &p.info);
@@ -1729,19 +1732,26 @@ static int spmv_in_scratch(void *scr, size_t scr_bytes, const int *d_row_ptr, co
     plan_carve(&p, static_cast<char *>(scr) + kNoallocStatsBytes);
     // row-aligned tiles split no row, so no owner slot is read: the error flag alone starts cleared
     st = p.info.row_aligned ? pfk_fill_zero(p.err, 256, stream) : plan_init(&p, d_row_ptr, stream);
-    if (st != PF_OK) return from_kernel_layer(st, "scratch workspace init");
+    if (st != PF_OK) {
+        st = from_kernel_layer(st, "scratch workspace init");
+        pfk_stream_sync(stream);
+        return st;
+    }
     st = pf_plan_execute(&p, d_row_ptr, d_col, d_val, d_x, d_y, stream);
-    if (st == PF_OK) st = pf_plan_check(&p, stream);  // synchronises: the scratch is free again on return
-    else pfk_stream_sync(stream);
+    if (st == PF_OK) st = pf_plan_check(&p, stream);  // synchronises
+    if (st != PF_OK) pfk_stream_sync(stream);
     return st;
 }
 
-// A one-shot call's plan lives for one product, so it is made in the device's scratch array where that is free and
-// large enough: no hipMalloc, hipFree, events or planning waits beyond the statistics' one.  us per call, with a
-// plan of its own -> in the scratch: 1448^2 5-point grid fp64 190 -> 107, 4096 rows of 16 100 -> 62, 2M power-law
-// rows 1012 -> 336 (no hybrid tables for one product), 20M rows of 2.5 (50M nnz) 532 -> 532.  Above kScratchNnz the
-// tables pay even once or the workspace may not fit; those calls, explicit variants, incomplete arguments (for their
-// error) and calls that find another thread in the scratch make a plan.
+// A one-shot call's plan lives for one product, so it is made in the device's scratch array where that is large
+// enough: no hipMalloc, hipFree, events or planning waits beyond the statistics' one.  us per call, with a plan of its
+// own -> in the scratch: 1448^2 5-point grid fp64 190 -> 107, 4096 rows of 16 100 -> 62, 2M power-law rows 1012 -> 336
+// (no hybrid tables for one product), 20M rows of 2.5 (50M nnz) 532 -> 532.  A call that finds another thread in the
+// scratch makes the same plan in an allocation of the scratch's size, so that y does not depend on other threads: that
+// plan's kernels are chosen by the row statistics alone, without what plan creation learns from the long rows and the
+// columns (hybrid plans, row groups beside long rows or for scattered columns), whose sums round otherwise.  Above
+// kScratchNnz the tables pay even once or the workspace may not fit; those calls, explicit variants and incomplete
+// arguments (for their error) make a plan.
 constexpr long long kScratchNnz = 64LL << 20;
 
 int pf_spmv(const int *d_row_ptr, const int *d_col, const void *d_val, const void *d_x, void *d_y, int m, int n,
@@ -1753,13 +1763,17 @@ int pf_spmv(const int *d_row_ptr, const int *d_col, const void *d_val, const voi
     if (variant == PF_AUTO && m > 0 && nnz > 0 && nnz <= kScratchNnz && d_row_ptr && d_col && d_val && d_x && d_y &&
         check_matrix_args(d_row_ptr, d_col, m, n, nnz, dtype, variant) == PF_OK && aligned16(d_val) &&
         pfk_get_device(&dev) == PF_OK && dev >= 0 && dev < kNoallocDevices && pfk_scratch(&scr, &scr_bytes) == PF_OK) {
+        warm_queues();
         std::unique_lock<std::mutex> lock(g_noalloc_mu[dev], std::try_to_lock);
-        if (lock.owns_lock()) {
-            warm_queues();
-            const int st = spmv_in_scratch(scr, scr_bytes, d_row_ptr, d_col, d_val, d_x, d_y, m, n, nnz, dtype, variant,
-                                           stream);
-            if (st != PF_ERR_UNSUPPORTED) return st;
+        void *own = nullptr;
+        if (!lock.owns_lock()) {
+            PF_TRY(pfk_malloc(&own, scr_bytes), "one-shot workspace");
+            scr = own;
         }
+        const int st = spmv_in_scratch(scr, scr_bytes, d_row_ptr, d_col, d_val, d_x, d_y, m, n, nnz, dtype, variant,
+                                       stream);
+        if (own) pfk_free(own);
+        if (st != PF_ERR_UNSUPPORTED) return st;
     }
     pf_plan *p = nullptr;
     int st = pf_plan_create(&p, d_row_ptr, d_col, m, n, nnz, dtype, variant, stream);

@@ -76,3 +76,41 @@ def test_threads_share_the_device():
     for t in threads:
         t.join(timeout=60)
     assert not any(t.is_alive() for t in threads) and not failures, failures
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("family,size", [(1, 300007), (3, 800000), (5, 40000)],
+                         ids=["scattered", "power-law", "dense-rows"])
+def test_y_does_not_depend_on_other_threads(family, size, dtype):
+    """Random values, whose sums depend on their order: calls that find another thread in the scratch give the bits of
+    a call that has it for itself.  Plans of these matrices take other kernels (row groups, long rows, hybrid)."""
+    rp, col, v = pf.synth_csr(family, seed=9, scale_n=size, dtypes=(dtype,))
+    m = len(rp) - 1
+    d = [dev(a) for a in (rp, col, v[dtype], pf.synth_x(family, m, seed=9, dtypes=(dtype,))[dtype])]
+    want = torch.full((m,), float("nan"), dtype=TORCH[dtype], device=DEV)
+    pf.spmv(*d, want, m, m, len(col), dtype)
+    assert_parity(rp, col, v[dtype], d[3].cpu().numpy(), want.cpu().numpy(), dtype, what=f"{family} {dtype} alone")
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    start, failures = threading.Barrier(len(streams)), []
+
+    def worker(k):
+        try:
+            y = [torch.full((m,), float("nan"), dtype=TORCH[dtype], device=DEV) for _ in range(6)]
+            torch.cuda.synchronize()
+            start.wait(timeout=60)
+            for out in y:
+                pf.spmv(*d, out, m, m, len(col), dtype, "auto", streams[k])
+            for it, out in enumerate(y):
+                if not torch.equal(out, want):
+                    failures.append((k, it, int((out != want).sum())))
+        except Exception as e:
+            failures.append((k, repr(e)))
+            start.abort()
+
+    threads = [threading.Thread(target=worker, args=(k,)) for k in range(len(streams))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert not any(t.is_alive() for t in threads) and not failures, failures
