@@ -247,11 +247,11 @@ int pfk_plan_scan(const int *row_ptr, const int *col, int m, int n, long long nn
 #define PFK_BAND_SAMPLE 16
 int pfk_band_stats(const int *row_ptr, const int *col, int m, unsigned long long *out, void *stream);
 
-/* Columns of neighbouring rows: over a sample of the rows, out[0] = the entries whose column lies within
- * PFK_SCATTER_NEAR of the next row's entry of the same position, out[1] = the entries compared.  row_ptr and col as
- * checked at planning; `out`: 2 device words.  Asynchronous on `stream`. */
+/* Columns of neighbouring rows: over a sample of the rows, out[0] = the entries whose column lies within `near` of
+ * the next row's entry of the same position, out[1] = the entries compared.  row_ptr and col as checked at planning;
+ * `out`: 2 device words.  Asynchronous on `stream`. */
 #define PFK_SCATTER_NEAR 1024
-int pfk_scatter_stats(const int *row_ptr, const int *col, int m, int nnz, unsigned int *out, void *stream);
+int pfk_scatter_stats(const int *row_ptr, const int *col, int m, int nnz, int near, unsigned int *out, void *stream);
 
 /* Tile descriptors of ADAPTIVE (merged=1) / FLAT (merged=0) for every tile:
  * d_out[8*t + 0..5] = first row, row count, first nnz, end nnz, head split, tail split. */

@@ -2396,7 +2396,7 @@ constexpr int kBandStatsWg = 512;
 
 // How far neighbouring rows' columns lie apart: over kScatterRows rows spread
 // over the matrix, their first kScatterPer entries, out[0] = the entries whose column
-// lies within PFK_SCATTER_NEAR of the next row's entry of the same position,
+// lies within `dist` columns of the next row's entry of the same position,
 // out[1] = the entries compared.  A stencil or a band has nearly all of them
 // near, whatever block of rows of it this is; random columns few.  One
 // workgroup, 7.7 us once per plan that asks (a lane per row, 2048 rows: 41.4).
@@ -2405,7 +2405,7 @@ constexpr int kScatterRows = 256;
 constexpr int kScatterPer = 16;  // entries of a row, a lane each: two latencies a pass, four passes in flight
 
 __global__ __launch_bounds__(kScatterBS) void k_scatter_stats(const int *__restrict__ rp, const int *__restrict__ col,
-                                                              int m, int nnz, unsigned int *__restrict__ out)
+                                                              int m, int nnz, int dist, unsigned int *__restrict__ out)
 {
     __shared__ unsigned int s_n[2];
     const int tid = threadIdx.x;
@@ -2419,7 +2419,7 @@ __global__ __launch_bounds__(kScatterBS) void k_scatter_stats(const int *__restr
         if (r + 1 >= m) continue;
         const int a = min(max(rp[r], 0), nnz), b = min(max(rp[r + 1], a), nnz), c = min(max(rp[r + 2], b), nnz);
         if (k >= min(b - a, c - b)) continue;
-        near += llabs((long long)col[a + k] - col[b + k]) <= PFK_SCATTER_NEAR ? 1u : 0u;
+        near += llabs((long long)col[a + k] - col[b + k]) <= dist ? 1u : 0u;
         ++all;
     }
     const auto add = [](unsigned int x, unsigned int y) { return x + y; };
@@ -5113,10 +5113,10 @@ int pfk_band_stats(const int *row_ptr, const int *col, int m, unsigned long long
     return PF_OK;
 }
 
-int pfk_scatter_stats(const int *row_ptr, const int *col, int m, int nnz, unsigned int *out, void *stream)
+int pfk_scatter_stats(const int *row_ptr, const int *col, int m, int nnz, int near, unsigned int *out, void *stream)
 {
-    if (!row_ptr || !out || m < 0 || nnz < 0 || (nnz > 0 && !col)) return PF_ERR_INVALID;
-    hipLaunchKernelGGL(k_scatter_stats, dim3(1), dim3(kScatterBS), 0, S(stream), row_ptr, col, m, nnz, out);
+    if (!row_ptr || !out || m < 0 || nnz < 0 || near < 0 || (nnz > 0 && !col)) return PF_ERR_INVALID;
+    hipLaunchKernelGGL(k_scatter_stats, dim3(1), dim3(kScatterBS), 0, S(stream), row_ptr, col, m, nnz, near, out);
     PFK_LAUNCHED("k_scatter_stats");
     return PF_OK;
 }

@@ -341,7 +341,7 @@ int row_group_lanes(const pf_row_stats &s)
 //     99; 262144 x 128, 403 MB, 239 against 192 for 2048-nnz tiles);
 //   * more rows, none longer than 64, of 7 to 16 nnz on average, values and
 //     columns within 64 MB, or 88 MiB for 12 nnz per row and more: row groups
-//     too in a plan that finds the columns scattered (scattered_columns), where
+//     too in a plan that finds the columns scattered (near_share), where
 //     every gather is a line of its own whoever makes it and a tile's barriers
 //     and LDS round trip hold the gathers back.  Where rows follow each other's
 //     columns the tiles' gathers share lines and row groups lose: 9-point
@@ -352,7 +352,9 @@ int row_group_lanes(const pf_row_stats &s)
 //     (fp64).  The lines: 16-nnz rows over 86 MB (450000, fp64) take 44.7 us with
 //     16 lanes against 47.2 for tiles, 90 MB (700000, fp32) 53.6 against 56.7,
 //     102 MB (800000, fp32) 66.0 against 64.1, 115 MB (600000, fp64) 68.0 against
-//     69.0, 134 MB (700000, fp64) 92 against 84; 24-nnz rows 49.7 against 48.3;
+//     69.0, 134 MB (700000, fp64) 92 against 84; 24-nnz rows 49.7 against 48.3, 27-point
+//     stencils 31.3 against 27.4.  fp16, 8 lanes against 2048-nnz tiles: 92 MB (960001
+//     rows of 16) 69.2 and 71.1, 125 MB 93.3 and 94.9, 12-nnz rows 94 MB 72.6 and 72.9;
 //   * no row longer than PFK_ALIGN_ROW_MAX, or fp16 values (FLAT only): FLAT
 //     (1024 nnz per tile for fp64, 2048 for fp32 / fp16 or for rows of under
 //     4 nnz on average), row-aligned when the rows fit: one launch per call;
@@ -1006,10 +1008,34 @@ int try_hybrid(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream,
 // where the table or the rules would cut every row at tile edges.  The short rows hold 12 nnz or more on average
 // and at most 128 (8 passes of a group), the long rows 1024 or more on average and at most 2^16, values and
 // columns are within 128 MB and x within one XCD's L2.  Measured, us per call, against the tiles: rows of 8-64 nnz
-// with a thousandth of long ones, fp64: 20,011 rows 8.0 against 11.6, 60,000 rows 20 against 25, 120,011 (99 MB)
-// 39 against 46, 200,001 (221 MB) 83 against 79; fp32: 120,011 rows 30 against 37, 200,001 (147 MB) 58 against 60,
-// 300,000 (280 MB) 107 against 96.  Short rows of 4 nnz (power law) take 55 against 24.
-bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanScan *scan)
+// with a thousandth of long ones, random columns, fp64: 20,011 rows 8.0 against 11.6, 60,000 rows 20 against 25,
+// 120,011 (99 MB) 39 against 46, 200,001 (221 MB) 83 against 79; fp32: 120,011 rows 30 against 37, 200,001 (147 MB)
+// 58 against 60, 300,000 (280 MB) 107 against 96.  Short rows of 4 nnz (power law) take 55 against 24.
+//
+// The columns decide too where `ask` says so.  `near`: where neighbouring rows' columns lie together (stencils,
+// narrow bands) the tiles' gathers share lines, and a tile sums rows of up to 16 nnz with a lane each.  Such matrices keep their
+// tiles over 40 MB of values and columns in fp64 and 50 MB in fp32 and fp16, and with short rows of 16 nnz or fewer on
+// average at any size (fp16: over 20 MB).  With 20 rows of 20,000 nnz, us per call, row groups and 2048-nnz tiles:
+//   25-point 2-D stencil  fp64  35 MB 17.4, 17.3   49 MB 20.9, 20.8   62 MB 25.8, 24.1  113 MB 46.9, 37.2
+//                         fp32  42 MB 16.0, 19.1   55 MB 20.0, 21.9   75 MB 27.0, 27.0   99 MB 34.6, 33.0
+//                         fp16  41 MB 19.6, 22.0   56 MB 24.2, 25.8   74 MB 30.7, 31.2   92 MB 38.4, 36.8
+//   18 within +-300       fp64  35 MB 19.2, 19.6   49 MB 25.3, 23.8    fp32  42 MB 19.5, 20.7   55 MB 25.7, 24.0
+//   27-point 3-D stencil  fp64  50 MB 20.4, 20.8   81 MB 31.8, 28.2  110 MB 42.7, 35.7
+//   49-point 2-D stencil  fp32  41 MB 14.5, 16.1   55 MB 19.0, 18.6   99 MB 30.5, 27.2
+//   16 within +-300       fp64  17 MB 13.9, 11.8   fp32  23 MB 13.7, 11.6   fp16  17 MB 9.9, 11.3   25 MB 13.2, 12.7
+// Columns that lie further apart are as good as random ones: 24 within +-3000, fp64, 112 MB 47.7, 51.9.
+//
+// `band`: where x is over 2.2 MB (fp32, fp16: 2.7): random columns then miss an L2 that the values pass
+// through, and the row groups, whose waves wait for every miss, lose to the tiles' deeper batches; in a band the x
+// in use is small whatever its length.  fp64, random: rows of 20, x 2.0 MB 39.0, 41.9   2.6 MB 54.8, 50.8   3.2 MB
+// 72.7, 60.2; of 30, 2.13 MB 54.1, 56.7   2.48 MB 65.6, 64.2; fp32 rows of 18, 2.0 MB 52.5, 54.3   2.67 MB 73.2, 69.2
+// 3.33 MB 102.8, 83.4; fp64, 24 within +-20,000, x 3.67 MB 67.2, 72.6.  Rows of up to 20 nnz, whose second pass leaves
+// most lanes idle, lose there in a band too (18 within +-3000, fp64, x 3.56 MB 54.2, 49.4): tiles without asking.
+struct BesideAsk {
+    bool near = false, band = false;
+};
+
+bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanScan *scan, BesideAsk *ask)
 {
     if (!scan || !scan->list || s.n_long_rows < 1 || scan->listed != s.n_long_rows || scan->host_n != scan->listed)
         return false;
@@ -1017,9 +1043,14 @@ bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanS
     for (long long k = 0; k < scan->host_n; ++k)
         long_nnz += scan->host[(size_t)(4 * k + 2)] - (long long)scan->host[(size_t)(4 * k + 1)];
     const long long short_nnz = s.nnz - long_nnz, short_rows = s.m - s.n_long_rows;
+    const long long stream = s.nnz * (value_bytes(dtype) + 4);
+    const long long near_max = short_nnz <= 16 * short_rows ? (dtype == PF_F16 ? 20000000LL : 0)
+                                                            : (dtype == PF_F64 ? 40000000LL : 50000000LL);
+    ask->near = stream > near_max;
+    ask->band = n * value_bytes(dtype) > (dtype == PF_F64 ? 2200000 : 2700000);
+    if (ask->band && short_nnz <= 20 * short_rows) return false;
     return s.max_row_len <= (1LL << 16) && long_nnz >= 1024 * s.n_long_rows && s.max_short_row_len <= 128 &&
-           short_nnz >= 12 * short_rows && s.nnz * (value_bytes(dtype) + 4) <= kVectorLongBytesMax &&
-           n * value_bytes(dtype) <= kXcdL2Bytes;
+           short_nnz >= 12 * short_rows && stream <= kVectorLongBytesMax && n * value_bytes(dtype) <= kXcdL2Bytes;
 }
 
 // The list of a row-groups-beside-long-rows plan on the device, longest row first (the long rows start with the
@@ -1086,21 +1117,22 @@ int try_band(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream, P
     return PF_OK;
 }
 
-// Whether fewer than a quarter of the sampled entries lie within PFK_SCATTER_NEAR columns of the next row's (random
-// columns over 300,000: 2%; stencils and bands: nearly all of them).  Synchronises `stream`.
-int scattered_columns(const int *d_row_ptr, const int *d_col, int m, int nnz, void *stream, PlanTimer *timer, bool *yes)
+// The share of the sampled entries that lie within `near` columns of the next row's (1 where none were compared).
+// Random columns over 300,000, 1024 near: 2%; stencils and bands: nearly all of them.  Synchronises `stream`.
+int near_share(const int *d_row_ptr, const int *d_col, int m, int nnz, int near, void *stream, PlanTimer *timer,
+               double *share)
 {
     unsigned int *d = nullptr;
     unsigned int h[2] = {0, 0};
     PF_TRY(pfk_malloc(reinterpret_cast<void **>(&d), sizeof h), "column statistic");
     if (timer) timer->start(stream);
-    int st = pfk_scatter_stats(d_row_ptr, d_col, m, nnz, d, stream);
+    int st = pfk_scatter_stats(d_row_ptr, d_col, m, nnz, near, d, stream);
     if (st == PF_OK) st = pfk_memcpy_d2h(h, d, sizeof h, stream);
     if (st == PF_OK) st = pfk_stream_sync(stream);
     if (st == PF_OK && timer) timer->stop(stream);
     pfk_free(d);
     if (st != PF_OK) return from_kernel_layer(st, "column statistic");
-    *yes = 4ull * h[0] < h[1];
+    *share = h[1] > 0 ? (double)h[0] / (double)h[1] : 1.0;
     return PF_OK;
 }
 
@@ -1118,18 +1150,28 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
     const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid, &allow_beside, &scattered);
     bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && allow_hybrid;
     if (st != PF_OK) return st;
-    bool beside = false;  // row groups beside long rows
-    if (allow_beside && tile <= 0 && !(want_hybrid && hybrid_candidate(s, n, dtype, info, d_col)) &&
-        vector_long_rule(s, n, dtype, scan)) {
+    double near = 0.0;
+    BesideAsk ask;
+    bool beside = allow_beside && tile <= 0 && d_col && !(want_hybrid && hybrid_candidate(s, n, dtype, info, d_col)) &&
+                  vector_long_rule(s, n, dtype, scan, &ask);  // row groups beside long rows
+    if (beside && ask.near) {  // tiles where half the entries lie within 8 or 16 lines of x of the next row's
+        const int st2 = near_share(d_row_ptr, d_col, m, nnz, dtype == PF_F16 ? 1024 : 256, stream, timer, &near);
+        if (st2 != PF_OK) return st2;
+        beside = near < 0.5;
+    }
+    if (beside && ask.band) {  // random columns: 15-20% within n / 64; a band: most
+        const int st2 = near_share(d_row_ptr, d_col, m, nnz, n / 64, stream, timer, &near);
+        if (st2 != PF_OK) return st2;
+        beside = near >= 0.5;
+    }
+    if (beside) {
         const int st2 = finish_info(s, dtype, PF_FLAT, PFK_VECTOR_LONG_LANES, &info);
         if (st2 != PF_OK) return st2;
-        beside = true;
         want_hybrid = false;
     }
-    if (scattered > 0 && tile <= 0 && d_col) {
-        bool yes = false;
-        int st2 = scattered_columns(d_row_ptr, d_col, m, nnz, stream, timer, &yes);
-        if (st2 == PF_OK && yes) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
+    if (scattered > 0 && tile <= 0 && d_col) {  // row groups where under a quarter of the entries are near
+        int st2 = near_share(d_row_ptr, d_col, m, nnz, PFK_SCATTER_NEAR, stream, timer, &near);
+        if (st2 == PF_OK && near < 0.25) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
         if (st2 != PF_OK) return st2;
     }
     pf_plan *p = new pf_plan();

@@ -77,6 +77,56 @@ def test_rule_refuses(what, change):
     assert_parity(rp, col, val, x, y, "f64", exact=True, what=what)
 
 
+def _stencil_with_long_rows(points, side, nlong, length, seed=3):
+    """`points` columns a row around it on a side x side x side (27) or side x side grid (16), random ones (0: 27
+    a row; -w: 24 a row within w of it, of `side` rows), and nlong rows of `length` random columns among them."""
+    rng = np.random.default_rng(seed)
+    if points < 0:
+        off = np.zeros(0, dtype=np.int64)
+    elif points == 27:
+        d = np.array([-1, 0, 1])
+        off = (side * side * d[:, None, None] + side * d[None, :, None] + d[None, None, :]).ravel()
+    else:
+        d = np.arange(-1, 3)
+        off = (side * d[:, None] + d[None, :]).ravel()
+    n = side if points < 0 else side ** 3 if points in (0, 27) else side ** 2
+    if points < 0:
+        cols = np.sort((np.arange(n)[:, None] + rng.integers(points, 1 - points, (n, 24))) % n, axis=1)
+    else:
+        cols = np.sort(rng.integers(0, n, (n, 27)), axis=1) if points == 0 else np.arange(n)[:, None] + off[None, :]
+    ok = (cols >= 0) & (cols < n)
+    at = np.sort(rng.choice(n, nlong, replace=False))
+    ok[at] = False
+    lens = ok.sum(1)
+    pieces, start = [], 0
+    short = np.concatenate([[0], np.cumsum(lens)])
+    flat = cols[ok]
+    for r in at:
+        pieces += [flat[short[start]:short[r]], np.sort(rng.choice(n, length, replace=False))]
+        start = r
+    pieces.append(flat[short[start]:])
+    lens[at] = length
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    return rp, np.concatenate(pieces).astype(np.int32), n
+
+
+@pytest.mark.parametrize("points,side,dtype,groups", [
+    (27, 56, "f64", False), (27, 56, "f32", True),    # 57 MB of values and columns, 38 MB
+    (27, 63, "f32", False), (27, 63, "f16", True),    # 54 MB, 41 MB
+    (0, 56, "f64", True), (0, 63, "f32", True),       # random columns at any size within 2.2 MB of x
+    (-150000, 300007, "f64", False), (-150000, 300007, "f32", True), (-15000, 300007, "f64", True),  # 2.4 MB, 1.2 MB
+    (16, 150, "f64", False), (16, 150, "f32", False), (16, 150, "f16", True), (16, 480, "f16", False),
+])
+def test_columns_decide_beside_long_rows(points, side, dtype, groups):
+    """Long rows among stencils: tiles over the rule's bytes, and at any size where the rows are short; among random
+    columns over a large x: tiles, unless they lie in a band."""
+    rp, col, n = _stencil_with_long_rows(points, side, 8, 9000)
+    val, x = oracle.initvec(len(col), NP[dtype]), oracle.initvec(n, NP[dtype])
+    y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
+    assert (info["variant_name"], info["tile"]) == ("flat", 16 if groups else 2048), info
+    assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{points} {side} {dtype}")
+
+
 def test_special_values_and_graph_replay():
     rp, col, n = _matrix("adjacent")
     rng = np.random.default_rng(2)
