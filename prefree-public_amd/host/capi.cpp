@@ -1004,6 +1004,23 @@ int try_hybrid(pf_plan *p, const int *d_row_ptr, const int *d_col, void *stream,
     return PF_OK;
 }
 
+// Bytes of x up to which row groups of scattered columns pay where those are random over all of x (see auto_choice):
+// past it the waves, which wait for every L2 miss, lose to the tiles' deeper batches.  In a band they pay at any size,
+// except for fp32 rows of 12 or 13 nnz (`both` false), whose 16 lanes only random columns keep busy.  us per call, row
+// groups and tiles: fp64 rows of 8, x 3.75 MB 28.0, 28.9   4.58 MB 38.2, 35.8   5.25 MB 48.7, 41.8; of 10, 2.33 MB
+// 21.3, 21.3   3.0 MB 28.3, 27.2   4.2 MB 46.4, 39.4; of 12, 4.17 MB 43.6, 44.9   5.06 MB 56.9, 56.4; fp32 of 8,
+// 2.81 MB 30.2, 32.4   3.44 MB 40.4, 39.0; of 10, 2.25 MB 31.0, 31.8   2.75 MB 39.8, 37.7; of 12, 2.29 MB 36.8, 37.6
+// 3.12 MB 54.1, 49.4; of 16, 2.84 MB 54.9, 57.6; fp16 of 10, 2.1 MB 50.3, 50.4; within +-20,000, fp64 of 8, 5.25 MB
+// 31.6, 36.9, fp32 of 10, 3.15 MB 38.1, 38.6, of 12, 1.46 MB 24.7, 23.1   3.79 MB 59.2, 52.9.
+long long scattered_x_max(const pf_row_stats &s, int dtype, bool *both)
+{
+    const long long m = s.m, nnz = s.nnz, any = 1LL << 62;
+    *both = dtype != PF_F32 || nnz < 12 * m || nnz >= 14 * m;
+    if (dtype == PF_F16 || nnz >= 14 * m || (dtype == PF_F64 && nnz >= 12 * m)) return any;
+    if (nnz >= 9 * m) return 2400000;
+    return dtype == PF_F64 ? 4200000 : 3200000;
+}
+
 // PF_AUTO: row groups beside long rows (k_vector_long), for a few long rows among short ones of middling length,
 // where the table or the rules would cut every row at tile edges.  The short rows hold 12 nnz or more on average
 // and at most 128 (8 passes of a group), the long rows 1024 or more on average and at most 2^16, values and
@@ -1159,8 +1176,8 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         if (st2 != PF_OK) return st2;
         beside = near < 0.5;
     }
-    if (beside && ask.band) {  // random columns: 15-20% within n / 64; a band: most
-        const int st2 = near_share(d_row_ptr, d_col, m, nnz, n / 64, stream, timer, &near);
+    if (beside && ask.band) {  // random columns: 15-35% within n / 32; a band: most
+        const int st2 = near_share(d_row_ptr, d_col, m, nnz, n / 32, stream, timer, &near);
         if (st2 != PF_OK) return st2;
         beside = near >= 0.5;
     }
@@ -1171,7 +1188,14 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
     }
     if (scattered > 0 && tile <= 0 && d_col) {  // row groups where under a quarter of the entries are near
         int st2 = near_share(d_row_ptr, d_col, m, nnz, PFK_SCATTER_NEAR, stream, timer, &near);
-        if (st2 == PF_OK && near < 0.25) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
+        bool groups = near < 0.25;
+        bool both = true;
+        const long long xb = (long long)n * value_bytes(dtype), xmax = scattered_x_max(s, dtype, &both);
+        if (st2 == PF_OK && groups && (xb > xmax || !both)) {
+            st2 = near_share(d_row_ptr, d_col, m, nnz, n / 32, stream, timer, &near);
+            groups = near >= 0.5 ? both : xb <= xmax;
+        }
+        if (st2 == PF_OK && groups) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
         if (st2 != PF_OK) return st2;
     }
     pf_plan *p = new pf_plan();

@@ -125,7 +125,9 @@ def test_auto_over_2_18_rows_of_middling_length(extra, longest, groups, dtype):
 @pytest.mark.parametrize("pattern,groups", [("9-point", False), ("random", True)])
 def test_auto_over_2_18_rows_looks_at_the_columns(pattern, groups, block, dtype):
     """9 columns a row: a stencil keeps its tiles, whole or as the second half of its rows (whose columns lie far from
-    its local row numbers); random columns take row groups."""
+    its local row numbers); random columns take row groups, but not in fp64 over the 4.2 MB of x of the half (24.2 us
+    in row groups, 21.0 in tiles)."""
+    groups = groups and not (block == 2 and dtype == "f64")
     side = 513 if block == 1 else 726
     n = side * side
     if pattern == "random":
@@ -144,3 +146,27 @@ def test_auto_over_2_18_rows_looks_at_the_columns(pattern, groups, block, dtype)
     y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
     assert (info["variant_name"], info["tile"] <= 32) == ("flat", groups), info
     assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{pattern} {block} {dtype}")
+
+
+@pytest.mark.parametrize("per,rows,dtype,random_groups,band_groups", [
+    (8, 400003, "f64", True, True), (8, 600001, "f64", False, True),     # x of 3.2 and 4.8 MB
+    (10, 290001, "f64", True, True), (10, 400003, "f64", False, True),   # 2.3 and 3.2 MB
+    (12, 400003, "f64", True, True),
+    (8, 600001, "f32", True, True), (8, 900001, "f32", False, True),     # 2.4 and 3.6 MB
+    (10, 500001, "f32", True, True), (10, 700001, "f32", False, True),   # 2.0 and 2.8 MB
+    (12, 300007, "f32", True, False), (12, 700001, "f32", False, False),
+    (16, 500001, "f32", True, True), (10, 700001, "f16", True, True),
+])
+def test_auto_over_2_18_rows_looks_at_the_size_of_x(per, rows, dtype, random_groups, band_groups):
+    """Scattered columns, random over all of x or within 20,000 of their row: row groups up to the rule's x, and over
+    it only in a band."""
+    rng = np.random.default_rng(9)
+    rp = (np.arange(rows + 1) * per).astype(np.int32)
+    val, x = oracle.initvec(rows * per, NP[dtype]), oracle.initvec(rows, NP[dtype])
+    for w, groups in ((0, random_groups), (20000, band_groups)):
+        cols = (np.arange(rows)[:, None] + rng.integers(-w, w + 1, (rows, per))) % rows if w else \
+            rng.integers(0, rows, (rows, per))
+        col = np.sort(cols, axis=1).astype(np.int32).ravel()
+        y, info = gpu_spmv(rp, col, val, x, "auto", dtype=dtype)
+        assert (info["variant_name"], info["tile"] <= 32) == ("flat", groups), (w, info)
+        assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{per} {rows} {dtype} {w}")
