@@ -153,8 +153,9 @@ int pf_plan_get_info(const pf_plan *plan, pf_plan_info *out);
 /* Row-aligned FLAT plans of fp64 / fp32 matrices whose x exceeds one XCD's L2 (4 MB) and whose columns lie
  * within +-w of their row for 85% or more of the nnz (w a power of two from 64 to 16384 that fits the band
  * kernel's LDS ring): planning measures the band (pfk_band_stats) and, for matrices of under 4 nnz per row
- * on average with w of 4096 or more, turns the band kernel on (not where a tuning-table row with hybrid 0 decides).  band 1 turns it on for any such plan, 0 off; PF_ERR_UNSUPPORTED for
- * a plan without a band.  Same y either way (bit for bit). */
+ * on average with w of 4096 or more, turns the band kernel on (not where a tuning-table row of variant
+ * "tiles" decides).  band 1 turns it on for any such plan, 0 off; PF_ERR_UNSUPPORTED for a plan without a band.  Same y
+ * either way (bit for bit). */
 int pf_plan_set_band(pf_plan *plan, int band);
 
 /* Planning time of a plan made by pf_plan_create / pf_plan_create_tuned: plan_ms is the wall time of the
@@ -245,16 +246,17 @@ int pf_plan_autotune(pf_plan *plan, const int *d_row_ptr, const int *d_col, cons
 
 /* Table for PF_AUTO, as written by the offline tuner (prefree-public_amd/tune/autotune.py).
  * Text, one row per line ('#' starts a comment):
- *   <class> <nnz_upper | -1> <rows> <f64|f32|f16> <adaptive|flat|prefree|auto> <tile> <run_tiles | 0>
+ *   <class> <nnz_upper | -1> <rows> <f64|f32|f16> <adaptive|flat|tiles|prefree|auto> <tile> <run_tiles | 0>
  *   <keep_cached> <ladder | 0> <hybrid 0|1>
  * (variant auto, tile 0: the matrices of that row keep PF_AUTO's built-in rules)
  * rows: the matrix's row-length class from its statistics — short (no row over 256 nnz, under 4 nnz
  * per row on average), regular (no row over 256 nnz), skewed (longer rows, under 16 nnz per row on
  * average), dense (longer rows, 16 or more on average) — or any.  The first row whose dtype and row
  * class match and whose bound exceeds the matrix's nnz decides (run 0: the built-in run rule; ladder
- * 0: the default ladder; hybrid 0: a FLAT plan stays split-row even with dense rows, and its tiles' kernel even with a band; flat 16 and a matrix with
- * rows over 256 nnz: row groups beside long rows, a workgroup each, where they pay, and the next row elsewhere).  Rows of the
- * older form <class> <nnz_upper> <dtype> <variant> <tile> <run> <keep> match any row class.
+ * 0: the default ladder; hybrid 0: a FLAT plan stays split-row even with dense rows; variant tiles: flat, but a
+ * plan with a band starts with its tiles' own kernel).  A "flat 16" row whose bound, class and type a later row repeats: for a matrix with rows over 256 nnz, row groups beside long rows, a
+ * workgroup each, where they pay, and the next row elsewhere.  Rows of the older form <class> <nnz_upper> <dtype>
+ * <variant> <tile> <run> <keep> match any row class.
  * NULL clears the table.  Without a call, the table named by $PREFREE_TUNING_TABLE is read once (an
  * empty value: none) or, when that is unset, tune/mi355x_tuning_table.txt beside the lib/ directory
  * of this library (the table measured on MI355X that ships with it).  Plans made before the call are

@@ -136,9 +136,11 @@ int choose_run(int tile, long long ntiles, long long resident)
 // One row per (size class, row-length class, value type): nnz below
 // `nnz_upper` (-1: no bound) and the matrix's row-length class select
 // (variant, tile, run_tiles, keep_cached, ladder, hybrid), or variant "auto"
-// (tile 0): the built-in rules.  A FLAT row of 16 lanes means, for a matrix with
-// long rows, row groups beside them where vector_long_rule takes them, and the
-// next row elsewhere.  The row-length
+// (tile 0): the built-in rules.  Variant "tiles" is FLAT whose plans start with
+// the tiles' own kernel where they have a band.  A FLAT row of 16 lanes whose bound, class
+// and type a later row repeats means, for a matrix with long rows, row groups
+// beside them where vector_long_rule takes them, and the next row elsewhere (a
+// repeated row could never be reached otherwise).  The row-length
 // classes are the cuts of the built-in rules below: "short" (every row <= 256
 // nnz, under 4 nnz per row on average), "regular" (every row <= 256 nnz),
 // "skewed" (longer rows, under 16 nnz per row on average), "dense" (longer
@@ -166,6 +168,7 @@ struct TableRow {
     std::string name;
     long long nnz_upper;
     int rows, dtype, variant, tile, run, keep, ladder, hybrid;
+    bool band;  // the band kernel may be on by default
 };
 
 std::mutex g_table_mu;
@@ -216,7 +219,8 @@ int load_table(const char *path, std::vector<TableRow> &out, std::string &why)
         r.name = w[0];
         r.rows = v2 ? parse_rows(w[2]) : kRowsAny;
         r.dtype = parse_dtype(w[2 + o]);
-        r.variant = parse_variant(w[3 + o]);
+        r.band = w[3 + o] != "tiles";
+        r.variant = r.band ? parse_variant(w[3 + o]) : PF_FLAT;
         try {
             size_t used = 0;
             const auto num = [&](const std::string &t) {
@@ -280,6 +284,7 @@ bool tile_supported(int variant, int dtype, int tile);
 struct Choice {
     int variant = PF_ADAPTIVE, tile = 0, run = 0, keep = -1, ladder = 0;
     bool hybrid = true;
+    bool band = true;    // the band kernel may be on by default
     bool beside = true;  // row groups beside long rows, where vector_long_rule takes them
     int scattered = 0;   // lanes per row of the row groups that a plan whose columns are scattered takes (0: none)
 };
@@ -290,12 +295,18 @@ bool table_choice(const pf_row_stats &s, int dtype, Choice &c)
     table_init_locked();
     const int rc = row_class(s);
     bool beside = false;
+    const auto repeated = [](const TableRow &r) {
+        const TableRow *end = g_table.data() + g_table.size();
+        return std::any_of(&r + 1, end, [&](const TableRow &l) {
+            return l.nnz_upper == r.nnz_upper && l.rows == r.rows && l.dtype == r.dtype;
+        });
+    };
     for (const TableRow &r : g_table) {
         if (r.dtype != dtype || (r.nnz_upper >= 0 && s.nnz >= r.nnz_upper)) continue;
         if (r.rows != kRowsAny && r.rows != rc) continue;
         if (r.variant == PF_AUTO) return false;  // this class keeps the built-in rules
         if (!tile_supported(r.variant, dtype, r.tile)) continue;
-        if (r.variant == PF_FLAT && r.tile == PFK_VECTOR_LONG_LANES && s.n_long_rows > 0) {
+        if (r.variant == PF_FLAT && r.tile == PFK_VECTOR_LONG_LANES && s.n_long_rows > 0 && repeated(r)) {
             beside = true;  // with long rows: beside them where vector_long_rule says so, else the next row
             continue;
         }
@@ -305,6 +316,7 @@ bool table_choice(const pf_row_stats &s, int dtype, Choice &c)
         c.keep = r.keep;
         c.ladder = r.ladder;
         c.hybrid = r.hybrid != 0;
+        c.band = r.band;
         c.beside = beside;
         return true;
     }
@@ -582,20 +594,15 @@ namespace {
 // Launch configuration of a plan for a validated matrix with known statistics
 // (host only, apart from occupancy queries): variant and tile (PF_AUTO
 // resolved), run length, x windows, workspace size.
-// `allow_hybrid` (optional) tells whether a FLAT plan of PF_AUTO may turn
-// hybrid: always, unless a tuning-table row says otherwise; `allow_beside`
-// whether row groups beside long rows may replace it.
+// `chosen` (optional) gets PF_AUTO's whole choice: what plan creation may make
+// of it from the long rows and the columns.
 int plan_info(const pf_row_stats &s, int n, int dtype, int variant, int tile, pf_plan_info *out,
-              bool *allow_hybrid = nullptr, bool *allow_beside = nullptr, int *scattered = nullptr)
+              Choice *chosen = nullptr)
 {
     Choice c;
-    if (allow_hybrid) *allow_hybrid = true;
-    if (allow_beside) *allow_beside = false;
+    c.beside = false;
     if (variant == PF_AUTO) {  // an explicit tile is kept only if the chosen variant has it
         c = auto_choice(s, dtype);
-        if (allow_hybrid) *allow_hybrid = c.hybrid;
-        if (allow_beside) *allow_beside = c.beside;
-        if (scattered) *scattered = c.scattered;
         variant = c.variant;
         if (tile <= 0 || !tile_supported(variant, dtype, tile)) tile = c.tile;
     }
@@ -616,6 +623,7 @@ int plan_info(const pf_row_stats &s, int n, int dtype, int variant, int tile, pf
     if (uses_row_map(info.variant, info.tile))
         info.x_windows = x_windows_rule(s, n, dtype, info.tile, info.row_aligned);
     *out = info;
+    if (chosen) *chosen = c;
     return PF_OK;
 }
 
@@ -1161,15 +1169,14 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
                void *stream, pf_plan **plan, const int *d_col = nullptr, const PlanScan *scan = nullptr,
                PlanTimer *timer = nullptr)
 {
-    bool allow_hybrid = true, allow_beside = false;
+    Choice c;
     pf_plan_info info;
-    int scattered = 0;
-    const int st = plan_info(s, n, dtype, variant, tile, &info, &allow_hybrid, &allow_beside, &scattered);
-    bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && allow_hybrid;
+    const int st = plan_info(s, n, dtype, variant, tile, &info, &c);
+    bool want_hybrid = (variant == PF_AUTO || variant == PF_FLAT) && tile <= 0 && c.hybrid;
     if (st != PF_OK) return st;
     double near = 0.0;
     BesideAsk ask;
-    bool beside = allow_beside && tile <= 0 && d_col && !(want_hybrid && hybrid_candidate(s, n, dtype, info, d_col)) &&
+    bool beside = c.beside && tile <= 0 && d_col && !(want_hybrid && hybrid_candidate(s, n, dtype, info, d_col)) &&
                   vector_long_rule(s, n, dtype, scan, &ask);  // row groups beside long rows
     if (beside && ask.near) {  // tiles where half the entries lie within 8 or 16 lines of x of the next row's
         const int st2 = near_share(d_row_ptr, d_col, m, nnz, dtype == PF_F16 ? 1024 : 256, stream, timer, &near);
@@ -1186,7 +1193,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         if (st2 != PF_OK) return st2;
         want_hybrid = false;
     }
-    if (scattered > 0 && tile <= 0 && d_col) {  // row groups where under a quarter of the entries are near
+    if (c.scattered > 0 && tile <= 0 && d_col) {  // row groups where under a quarter of the entries are near
         int st2 = near_share(d_row_ptr, d_col, m, nnz, PFK_SCATTER_NEAR, stream, timer, &near);
         bool groups = near < 0.25;
         bool both = true;
@@ -1195,7 +1202,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
             st2 = near_share(d_row_ptr, d_col, m, nnz, n / 32, stream, timer, &near);
             groups = near >= 0.5 ? both : xb <= xmax;
         }
-        if (st2 == PF_OK && groups) st2 = finish_info(s, dtype, PF_FLAT, scattered, &info);
+        if (st2 == PF_OK && groups) st2 = finish_info(s, dtype, PF_FLAT, c.scattered, &info);
         if (st2 != PF_OK) return st2;
     }
     pf_plan *p = new pf_plan();
@@ -1234,7 +1241,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         }
     }
     if (rc == PF_OK && d_col && !candidate) rc = try_band(p, d_row_ptr, d_col, stream, timer);
-    if (rc == PF_OK && !allow_hybrid) p->info.band_w = 0;  // a table row of plain tiles (pf_plan_set_band brings it back)
+    if (rc == PF_OK && !c.band) p->info.band_w = 0;  // a table row of plain tiles (pf_plan_set_band brings it back)
     if (rc == PF_OK && candidate) {
         rc = try_hybrid(p, d_row_ptr, d_col, stream, scan, timer);
         if (rc == PF_OK && !p->hybrid) {  // stays split-row: its workspace now

@@ -338,9 +338,8 @@ def write_table(best_by_dtype, thresholds, path, device=""):
                     lines.append(f"{cls} {bounds[cls]} {rows} {dtype} auto 0 0 0 0 1  # not measured")
                     continue
                 note = f"{b['mean_gbps']} GB/s mean; {b['why']}"
-                hybrid = 1 if rows == "short" else b["hybrid"]  # short rows: timed with the band kernel where it applies
                 lines.append(f"{cls} {bounds[cls]} {rows} {dtype} {b['variant']} {b['tile']} {b['run']} "
-                             f"{b['keep']} {b['ladder']} {hybrid}  # {note}")
+                             f"{b['keep']} {b['ladder']} {b['hybrid']}  # {note}")
     with open(path, "w") as f:
         f.write("\n".join(lines) + "\n")
 

@@ -135,15 +135,18 @@ def test_band_default_needs_a_wide_band():
 
 
 def test_table_row_of_plain_tiles(tmp_path):
-    """A table row with hybrid 0 keeps a banded plan's tiles; pf_plan_set_band switches the band on, same y."""
+    """A table row of variant "tiles" keeps a banded plan's tiles, one of variant "flat" has the band on, with the hybrid
+    column either way and in the older form; pf_plan_set_band switches it on, same y."""
     name, rp, col, n = CASES[0]
     m = len(rp) - 1
     val, x = oracle.initvec(len(col)), oracle.initvec(n)
     d = [dev(a) for a in (rp, col, val, x)]
     y = torch.full((m,), float("nan"), dtype=torch.float64, device="cuda:0")
-    for hybrid, band in ((0, 0), (1, 4096)):
-        t = tmp_path / f"table{hybrid}.txt"
-        t.write_text(f"t -1 short f64 flat 2048 0 0 0 {hybrid}\n")
+    for k, (row, band) in enumerate((("short f64 tiles 2048 0 0 0 0", 0), ("short f64 tiles 2048 0 0 0 1", 0),
+                                     ("short f64 flat 2048 0 0 0 0", 4096), ("short f64 flat 2048 0 0 0 1", 4096),
+                                     ("f64 flat 2048 0 0", 4096), ("f64 tiles 2048 0 0", 0))):
+        t = tmp_path / f"table{k}.txt"
+        t.write_text(f"t -1 {row}\n")
         pf.set_tuning_table(str(t))
         try:
             p = pf.Plan(d[0], d[1], m, n, len(col), "f64", "auto")
@@ -156,7 +159,7 @@ def test_table_row_of_plain_tiles(tmp_path):
                     p.set_band(True)
                 for _ in range(2):  # the first call records the map
                     p.execute(*d, y)
-                    assert_parity(rp, col, val, x, y.cpu().numpy(), "f64", exact=True, what=f"{name} {hybrid} {on}")
+                    assert_parity(rp, col, val, x, y.cpu().numpy(), "f64", exact=True, what=f"{name} {row} {on}")
 
 
 def test_band_plan_searching_every_call():

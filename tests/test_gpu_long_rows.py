@@ -77,6 +77,24 @@ def test_rule_refuses(what, change):
     assert_parity(rp, col, val, x, y, "f64", exact=True, what=what)
 
 
+@pytest.mark.parametrize("tail,tile", [("", 16), ("u -1 any f64 flat 2048 0 0 0 0\n", 16),
+                                       ("u -1 skewed f64 flat 2048 0 0 0 0\n", 2048)])
+def test_a_lone_table_row_of_16_lanes_means_row_groups(tmp_path, tail, tile):
+    """Rows under 12 nnz, where row groups beside long rows do not pay: a "flat 16" row is passed over only if a later
+    row repeats its bound, class and type."""
+    t = tmp_path / "lone.txt"
+    t.write_text("t -1 skewed f64 flat 16 0 0 0 0\n" + tail)
+    pf.set_tuning_table(str(t))
+    rng = np.random.default_rng(6)
+    lengths = rng.integers(0, 8, 3001)
+    lengths[1500] = 3000
+    rp, col = csr_from_lengths([int(v) for v in lengths], 70001, rng)
+    val, x = oracle.initvec(len(col)), oracle.initvec(70001)
+    y, info = gpu_spmv(rp, col, val, x, "auto")
+    assert (info["variant_name"], info["tile"]) == ("flat", tile), info
+    assert_parity(rp, col, val, x, y, "f64", exact=True, what="lone row")
+
+
 def _stencil_with_long_rows(points, side, nlong, length, seed=3):
     """`points` columns a row around it on a side x side x side (27) or side x side grid (16), random ones (0: 27
     a row; -w: 24 a row within w of it, of `side` rows), and nlong rows of `length` random columns among them."""
