@@ -35,7 +35,9 @@ each matrix.  A class's score:
      time and bytes the rules win over a fixed configuration.
 
 It writes
-  * a tuning table (text) that PF_AUTO reads: by default from
+  * a tuning table (text) that PF_AUTO reads, the config's pinned_rows (lines
+    between the size classes, or of plans that a class's few matrices cannot
+    place) at their places in it: by default from
     tune/mi355x_tuning_table.txt, else pf_set_tuning_table or
     $PREFREE_TUNING_TABLE — no source is generated or patched, no rebuild;
   * a results file (JSON) with every timing and counter reading.
@@ -322,17 +324,25 @@ def choose(per_class, band=0.01, guard=0.005, counter_fn=None, max_counted=3):
     return best
 
 
-def write_table(best_by_dtype, thresholds, path, device=""):
-    """The pf_set_tuning_table format: class nnz_upper rows dtype variant tile run keep ladder hybrid."""
+def write_table(best_by_dtype, thresholds, path, device="", pinned=None):
+    """The pf_set_tuning_table format: class nnz_upper rows dtype variant tile run keep ladder hybrid.  `pinned` (the
+    config's pinned_rows): table lines written `before` a "class/rows/dtype" row or `instead` of it."""
+    pinned = {k: (pinned or {}).get(k) or {} for k in ("before", "instead")}
     bounds = {"small": thresholds["small_upper"], "medium": thresholds["medium_upper"], "large": -1}
     lines = ["# preFree-MI355X tuning table, written by prefree-public_amd/tune/autotune.py"
-             + (f" on {device}" if device else ""),
+             + (f" on {device}" if device else "")
+             + (", with its config's pinned rows" if any(pinned.values()) else ""),
              "# class nnz_upper rows dtype variant tile run keep ladder hybrid"]
     for dtype, best in best_by_dtype.items():
         for rows in ROW_CLASSES:
             if not any((cls, rows) in best for cls in CLASSES):
                 continue
             for cls in CLASSES:   # first match by nnz: a size class without a row keeps the built-in rules
+                key = f"{cls}/{rows}/{dtype}"
+                for where in ("before", "instead"):
+                    lines += [line.strip() for line in pinned[where].get(key, "").splitlines() if line.strip()]
+                if key in pinned["instead"]:
+                    continue
                 b = best.get((cls, rows))
                 if not b:
                     lines.append(f"{cls} {bounds[cls]} {rows} {dtype} auto 0 0 0 0 1  # not measured")
@@ -532,7 +542,7 @@ def main():
                                     "matrices": [m for mats in per_class.values() for m in mats]}
     table = os.path.join(out_dir, cfg.get("output", {}).get("table_file", "tuning_table.txt"))
     res = os.path.join(out_dir, cfg.get("output", {}).get("results_file", "tuning_results.json"))
-    write_table(best_by_dtype, thresholds, table, device)
+    write_table(best_by_dtype, thresholds, table, device, cfg.get("pinned_rows"))
     with open(res, "w") as f:
         json.dump(results, f, indent=1)
     with open(os.path.join(out_dir, cfg.get("output", {}).get("summary_file", "tuning_summary.json")), "w") as f:

@@ -337,6 +337,31 @@ def test_committed_table_parses_and_names_the_row_classes(table):
             assert len(line) == 10 and line[2] in ("short", "regular", "skewed", "dense", "any"), line
 
 
+def test_committed_table_is_what_the_tuner_writes(tmp_path):
+    """The shipped table follows from the tuner's summary beside it and its config's pinned rows: running the tuner
+    again drops no row."""
+    import json
+    import os
+
+    import yaml
+    at = _autotune_module()
+    tune = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "prefree-public_amd", "tune")
+    with open(os.path.join(tune, "config.yaml")) as f:
+        cfg = yaml.safe_load(f)
+    with open(os.path.join(tune, "mi355x_tuning_summary.json")) as f:
+        summary = json.load(f)
+    best = {dt: {tuple(k.split("/")): b for k, b in r["classes"].items()} for dt, r in summary["dtypes"].items()}
+    out = tmp_path / "table.txt"
+    at.write_table(best, cfg["size_thresholds"], str(out), summary["device"], cfg["pinned_rows"])
+    with open(os.path.join(tune, "mi355x_tuning_table.txt")) as f:
+        assert f.read() == out.read_text()
+    keys = {f"{c}/{r}/{d}" for c in at.CLASSES for r in at.ROW_CLASSES for d in best}
+    for lines in cfg["pinned_rows"].values():
+        assert set(lines) <= keys
+    pinned = [line for lines in cfg["pinned_rows"].values() for text in lines.values() for line in text.splitlines()]
+    assert len(pinned) > 10 and all(line in out.read_text() for line in pinned)
+
+
 @pytest.mark.gpu
 def test_offline_tuner_runs_end_to_end(tmp_path):
     import subprocess
