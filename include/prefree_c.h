@@ -109,7 +109,9 @@ typedef struct pf_plan_info {
                              mode: rows of at least a few thousand nnz with sorted columns ("dense rows") summed by
                              x windows staged in LDS, shared by 128 rows at a time.  Long mode (long_tiles > 0):
                              the long rows cut into tiles of 1024 nnz dealt to the XCDs by their first column. */
-    long long dense_rows; /* hybrid plans: the rows summed apart (dense rows, or long rows in long mode) */
+    long long dense_rows; /* hybrid plans: the rows summed apart (dense rows, or long rows in long mode).  FLAT tile 16
+                             with hybrid 0 and dense_rows > 0: row groups beside that many rows over 256 nnz, each
+                             summed whole by a workgroup of 1024 lanes (ntiles and grid count all workgroups) */
     int x_halves;         /* hybrid plans: 1 = the runs' tiles are processed once per half of x, by XCDs 0-3 and
                              4-7, so each XCD's random gathers fall in half of x (chosen when x is 4-24 MB) */
     int long_tiles;       /* hybrid plans in long mode: tiles of the long rows; 0 otherwise */
@@ -137,7 +139,9 @@ const char *pf_last_error(void);
 int pf_row_stats_compute(const int *d_row_ptr, const int *d_col, int m, int n, long long nnz,
                          pf_row_stats *out, void *stream);
 
-/* Variant and tile selection from statistics (host only, no GPU call). */
+/* Variant and tile selection from statistics (host only, no GPU call).  pf_plan_create takes three more steps for
+ * PF_AUTO, which need the long rows or the columns: hybrid plans, row groups (FLAT 2..32) for rows of 7-16 nnz whose
+ * columns are scattered, and row groups beside long rows (FLAT 16 with pf_plan_info.dense_rows > 0). */
 int pf_select(const pf_row_stats *stats, int dtype, int variant, pf_plan_info *out);
 
 /* Analyse a device CSR, choose a variant (PF_AUTO) or honour the requested
@@ -239,7 +243,9 @@ typedef struct pf_tune_result {
     double default_us;  /* of the configuration the plan had before tuning */
     long long chunk_nnz; /* FLAT 1024/2048: XCD chunk of the chosen configuration (see pf_plan_info) */
     int ladder;         /* PREFREE: the chosen reduction ladder 1..5; 0 otherwise */
-    int hybrid;         /* 1 if the chosen configuration is the plan's own hybrid one */
+    int hybrid;         /* 1 if the chosen configuration is the plan's own and sums its long rows apart: hybrid, or
+                           row groups beside long rows.  pf_plan_create makes it again; pf_plan_create_tuned with
+                           (variant, tile) makes plain tiles or row groups */
 } pf_tune_result;
 int pf_plan_autotune(pf_plan *plan, const int *d_row_ptr, const int *d_col, const void *d_val, const void *d_x,
                      void *d_y, int reps, int flags, void *stream, pf_tune_result *result);

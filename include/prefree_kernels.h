@@ -75,7 +75,7 @@ typedef struct pfk_spmv_args {
      * PFK_DENSE_WINDOW(dtype) columns (pfk_dense_nwin, pfk_dense_width); the rows between them form runs, each cut into row-aligned
      * tiles of `tile` nnz (every run row holds at most PFK_ALIGN_ROW_MAX nnz).  ntiles counts the tiles
      * of all runs. */
-    const int *dense_rows;   /* [n_dense] row indices, ascending */
+    const int *dense_rows;   /* [n_dense] row indices, ascending (row groups: see PFK_VECTOR_LONG_LANES) */
     int n_dense;
     int n_win;               /* pfk_dense_nwin(n, dtype) */
     int n_runs;
@@ -131,6 +131,7 @@ typedef struct pfk_spmv_args {
        sums (rows of at most 16 nnz in nnz order, bit-identical to the recorded-rows kernel); band_w only
        decides what stays in LDS.  0 < band_w <= PFK_BAND_RING / 2. */
     int band_w;
+    size_t dense_rows_bytes; /* row groups beside long rows: bytes behind dense_rows, checked as the others are */
 } pfk_spmv_args;
 
 /* The band kernel: nnz per step (whole tiles of the row map), x entries of its LDS ring, and the band widths
@@ -143,9 +144,14 @@ typedef struct pfk_spmv_args {
 #define PFK_LONG_TILE 1024
 
 /* Row groups beside long rows (pfk_spmv_flat, tile = PFK_VECTOR_LONG_LANES, n_dense > 0): dense_rows lists the n_dense
- * rows over PFK_ALIGN_ROW_MAX nnz, each once, and holds a bitmap of them behind the list, bit r & 31 of word r >> 5 for
- * row r, (m + 31) / 32 words; a workgroup sums each of them whole and the row groups the others. */
+ * rows over PFK_ALIGN_ROW_MAX nnz, each once and in any order (the longest first starts the long ones early), and holds
+ * a bitmap of them behind the list, bit r & 31 of word r >> 5 for row r, (m + 31) / 32 words; a workgroup of
+ * PFK_VECTOR_LONG_BS lanes sums each of them whole and the row groups the others. */
 #define PFK_VECTOR_LONG_LANES 16
+#define PFK_VECTOR_LONG_BS 1024
+#define PFK_VECTOR_LONG_GRID(m, n_dense) (((long long)(m) * PFK_VECTOR_LONG_LANES + PFK_VECTOR_LONG_BS - 1) / \
+                                              PFK_VECTOR_LONG_BS + (n_dense))
+#define PFK_VECTOR_LONG_INTS(m, n_dense) ((long long)(n_dense) + ((long long)(m) + 31) / 32)
 
 /* Bytes of one split-row partial (head / tail slot): fp32 in the fp16 mode. */
 #define PFK_SLOT_BYTES(dtype) ((dtype) == 0 ? 8 : 4)

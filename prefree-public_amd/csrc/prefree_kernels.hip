@@ -3416,7 +3416,7 @@ __global__ __launch_bounds__(kBS) void k_vector(Args<T> a)
 // batch's x arrives (two batches by name, so that no register with a load in
 // flight is copied); lane partials, then the waves' trees and one over the
 // waves (fp32 error against 64 bits on 120,011 rows: the waves in order 9.6e-8).
-constexpr int kVecBS = 1024;
+constexpr int kVecBS = PFK_VECTOR_LONG_BS;
 constexpr int kVecU = 8;
 
 // fp64 takes 71 registers, one workgroup per CU; batches of 4 (57, two per CU) lose: 20,011 rows 8.0 -> 8.9 us.
@@ -4611,7 +4611,9 @@ int launch_vector(const pfk_spmv_args *a, void *stream)
                      PFK_VECTOR_LONG_LANES);
             return PF_ERR_INVALID;
         }
-        const long long lgrid = ((long long)a->m * a->tile + kVecBS - 1) / kVecBS + a->n_dense;
+        if (!room(a->dense_rows, a->dense_rows_bytes, PFK_VECTOR_LONG_INTS(a->m, a->n_dense) * 4, "long-row list"))
+            return PF_ERR_INVALID;
+        const long long lgrid = PFK_VECTOR_LONG_GRID(a->m, a->n_dense);
         hipLaunchKernelGGL((k_vector_long<T, PFK_VECTOR_LONG_LANES>), dim3((unsigned)lgrid), dim3(kVecBS), 0, S(stream),
                            r, a->dense_rows, a->n_dense);
         PFK_LAUNCHED("k_vector_long");

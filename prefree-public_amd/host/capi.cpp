@@ -425,7 +425,8 @@ bool tile_supported(int variant, int dtype, int tile)
 }
 
 // Workgroups launched: ADAPTIVE runs of run_tiles tiles, four waves per
-// workgroup, runs dealt evenly to the XCDs; row groups ntiles workgroups; one
+// workgroup, runs dealt evenly to the XCDs; row groups ntiles workgroups (beside
+// long rows too: of 1024 lanes, the long rows' among them); one
 // tile per workgroup otherwise (FLAT 1024/2048: tiles padded to whole rounds
 // of XCD chunks).
 void set_grid(pf_plan_info &r)
@@ -438,7 +439,7 @@ void set_grid(pf_plan_info &r)
     } else if (uses_row_map(r.variant, r.tile)) {
         r.grid = pfk_flat_grid(r.ntiles, r.tile, r.chunk_nnz);
     } else if (r.variant == PF_FLAT && PFK_ROW_GROUP_TILE(r.tile)) {
-        r.grid = r.ntiles;  // row groups: one workgroup per 256 lanes, by index
+        r.grid = r.ntiles;  // row groups, by index
     } else {
         r.grid = ((r.ntiles + kXcds - 1) / kXcds) * kXcds;
     }
@@ -583,8 +584,9 @@ struct pf_plan {
     void *long_part = nullptr;
     size_t long_tiles_bytes = 0, long_deal_bytes = 0, long_row_tiles_bytes = 0, long_part_bytes = 0;
     // row groups beside long rows: the rows over PFK_ALIGN_ROW_MAX nnz, longest first
-    int *long_rows = nullptr;  // its own allocation
+    int *long_rows = nullptr;  // its own allocation, the rows' bitmap behind them
     int n_long_rows = 0;
+    size_t long_rows_bytes = 0;
     // the runs' stream beside the caller's, and the events that fork and join it (see pfk_spmv_args)
     void *aux_stream = nullptr, *ev_fork = nullptr, *ev_join = nullptr;
 };
@@ -1083,7 +1085,7 @@ bool vector_long_rule(const pf_row_stats &s, long long n, int dtype, const PlanS
 int add_long_rows(pf_plan *p, const PlanScan &scan, void *stream)
 {
     const size_t count = (size_t)scan.host_n;
-    std::vector<int> order(count), rows(count + ((size_t)p->m + 31) / 32, 0);
+    std::vector<int> order(count), rows((size_t)PFK_VECTOR_LONG_INTS(p->m, count), 0);
     for (size_t k = 0; k < count; ++k) order[k] = (int)k;
     const auto len = [&](int k) { return scan.host[(size_t)(4 * k + 2)] - scan.host[(size_t)(4 * k + 1)]; };
     std::sort(order.begin(), order.end(), [&](int x, int y) {
@@ -1099,6 +1101,10 @@ int add_long_rows(pf_plan *p, const PlanScan &scan, void *stream)
     if (st == PF_OK) st = pfk_stream_sync(stream);
     if (st != PF_OK) return from_kernel_layer(st, "long-row list");
     p->n_long_rows = (int)count;
+    p->long_rows_bytes = rows.size() * sizeof(int);
+    p->info.dense_rows = (long long)count;
+    p->info.ntiles = PFK_VECTOR_LONG_GRID(p->m, count);  // workgroups
+    set_grid(p->info);
     return PF_OK;
 }
 
@@ -1662,6 +1668,7 @@ int pf_plan_execute(pf_plan *plan, const int *d_row_ptr, const int *d_col, const
     a.ovf_cap = plan->info.row_aligned ? (int)std::min<long long>(PFK_ALIGN_ROW_MAX, plan->stats.max_row_len) : 0;
     a.dense_rows = plan->long_rows;
     a.n_dense = plan->n_long_rows;
+    a.dense_rows_bytes = plan->long_rows_bytes;
     a.band_w = a.row_map ? plan->info.band_w : 0;  // used once the row map is recorded; never without one
     const int dt = plan->info.dtype;
     if (plan->hybrid) {
@@ -2016,7 +2023,7 @@ int pf_plan_autotune(pf_plan *plan, const int *d_row_ptr, const int *d_col, cons
     best.keep_cached = plan->info.keep_cached;
     best.chunk_nnz = plan->info.chunk_nnz;
     best.ladder = plan->info.variant == PF_PREFREE ? plan->info.ladder : 0;
-    best.hybrid = plan->info.hybrid;
+    best.hybrid = plan->info.hybrid || plan->n_long_rows > 0 ? 1 : 0;
     best.us = base_us;
     best.default_us = base_us;
     best.candidates = 1;

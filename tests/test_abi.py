@@ -379,6 +379,18 @@ def test_row_map_and_schedule_sizes_checked():
     assert K.pfk_spmv_flat(pf.F64, ctypes.byref(a), None) == 1  # lists shorter than an even share
 
 
+@pytest.mark.parametrize("field,value,what", [("dense_rows_bytes", (3 + 32) * 4 - 1, b"long-row list"),
+                                              ("dense_rows_bytes", 3 * 4, b"long-row list"),
+                                              ("dense_rows", None, b"the rows' list"), ("tile", 8, b"the rows' list")])
+def test_row_groups_beside_long_rows_check_their_list(field, value, what):
+    # the list of 3 rows and a bitmap of m = 1000 rows (32 words) behind it
+    K = pf.klib()
+    a = _args(tile=16, row_aligned=1, dense_rows=0x10000, n_dense=3, dense_rows_bytes=(3 + 32) * 4)
+    setattr(a, field, value)
+    assert K.pfk_spmv_flat(pf.F64, ctypes.byref(a), None) == 1
+    assert what in K.pfk_last_error()
+
+
 def test_adaptive_owner_table_size_checked():
     K = pf.klib()
     a = _args(tile=512, owner_bytes=10)

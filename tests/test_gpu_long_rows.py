@@ -51,6 +51,8 @@ def test_long_rows_beside_row_groups(name, dtype):
     kv, kx = oracle.initvec(len(col), NP[dtype]), oracle.initvec(n, NP[dtype])
     y, info = gpu_spmv(rp, col, kv, kx, "auto", dtype=dtype)
     assert (info["variant_name"], info["tile"], info["hybrid"]) == ("flat", 16, 0), info
+    nlong = len(LONG[name])
+    assert info["dense_rows"] == nlong and info["ntiles"] == info["grid"] == (3001 * 16 + 1023) // 1024 + nlong, info
     assert_parity(rp, col, kv, kx, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{name}/kat")
     rng = np.random.default_rng(1)
     val = rng.uniform(-1, 1, len(col)).astype(NP[dtype])
@@ -93,6 +95,24 @@ def test_a_lone_table_row_of_16_lanes_means_row_groups(tmp_path, tail, tile):
     y, info = gpu_spmv(rp, col, val, x, "auto")
     assert (info["variant_name"], info["tile"]) == ("flat", tile), info
     assert_parity(rp, col, val, x, y, "f64", exact=True, what="lone row")
+
+
+def test_autotune_tells_the_plan_from_plain_row_groups():
+    """Where the plan's own row groups beside long rows win, the result says so; FLAT 16 by name has no long rows."""
+    rp, col, n = _matrix("largest")
+    m, nnz = len(rp) - 1, len(col)
+    d = [dev(a) for a in (rp, col, oracle.initvec(nnz), oracle.initvec(n))]
+    y = torch.full((m,), float("nan"), dtype=torch.float64, device=DEV)
+    want = oracle.spmv_serial(rp, col, oracle.initvec(nnz), oracle.initvec(n))
+    with pf.Plan(d[0], d[1], m, n, nnz) as p:
+        assert (p.info.tile, p.info.dense_rows) == (16, len(LONG["largest"]))
+        r = p.autotune(*d, y, reps=5)
+        assert r["hybrid"] == (1 if p.info.dense_rows else 0) and (r["variant"], r["tile"]) == (p.info.variant, p.info.tile)
+        assert np.array_equal(y.cpu().numpy(), want)
+    with pf.Plan(d[0], d[1], m, n, nnz, "f64", "flat", 16) as p:
+        assert (p.info.tile, p.info.dense_rows, p.info.grid) == (16, 0, (16 * m + 255) // 256)
+        p.execute(*d, y)
+        assert np.array_equal(y.cpu().numpy(), want)
 
 
 def _stencil_with_long_rows(points, side, nlong, length, seed=3):
