@@ -174,7 +174,9 @@ int pf_plan_set_run_tiles(pf_plan *plan, int run_tiles);
 int pf_plan_set_keep_cached(pf_plan *plan, int keep_cached);
 /* FLAT 1024/2048 only: 1 = row-aligned tiles (chosen at planning when every
  * row holds at most 256 nnz), 0 = nnz tiles with split rows combined by a
- * second kernel.  Both give the same y. */
+ * second kernel.  Both give the same y.  This and the next two settings take a plan whose row groups PF_AUTO chose by
+ * the long rows or the columns back to the tiles that those replaced (the first call allocates their workspace and
+ * synchronises the default stream; y then within rounding of the row groups'). */
 int pf_plan_set_row_aligned(pf_plan *plan, int row_aligned);
 /* Split-row FLAT 1024/2048 only: 1 = the plan's first call records, with the row map, which eighth of x
  * each tile starts in, and later calls deal the tiles to the 8 XCDs by it (long rows then read one XCD's
@@ -195,7 +197,8 @@ int pf_plan_set_chunk_nnz(pf_plan *plan, long long chunk_nnz);
  * The tile size (pf_plan_create_tuned: 512 or 1024 nnz) is the reference's P_NNZ 4 or 8. */
 int pf_plan_set_ladder(pf_plan *plan, int ladder);
 /* Plans that PF_AUTO made hybrid (pf_plan_info.hybrid): 0 = split-row FLAT tiles instead, 1 = back to
- * hybrid.  Both give y within rounding of each other (the dense rows' partial sums differ in order).  A hybrid
+ * hybrid, PF_ERR_UNSUPPORTED for a plan that was not made hybrid (PF_AUTO leaves matrices to their tiles where the
+ * tuning table says hybrid 0; PF_FLAT with the default tile does not ask the table).  Both give y within rounding of each other (the dense rows' partial sums differ in order).  A hybrid
  * plan is built without the split-row workspace (pf_plan_info.workspace_bytes): the first switch to 0
  * allocates and initialises it on the default stream and synchronises that stream. */
 int pf_plan_set_hybrid(pf_plan *plan, int hybrid);

@@ -587,6 +587,7 @@ struct pf_plan {
     int *long_rows = nullptr;  // its own allocation, the rows' bitmap behind them
     int n_long_rows = 0;
     size_t long_rows_bytes = 0;
+    pf_plan_info tiles{};  // the FLAT tiles that row groups chosen by the long rows or columns replaced (tile 0: none)
     // the runs' stream beside the caller's, and the events that fork and join it (see pfk_spmv_args)
     void *aux_stream = nullptr, *ev_fork = nullptr, *ev_join = nullptr;
 };
@@ -733,6 +734,32 @@ int plan_add_split(pf_plan *p)
         return from_kernel_layer(rc, "split-row workspace");
     }
     p->ws_split = w;
+    return PF_OK;
+}
+
+// The tiles that the settings of FLAT 1024 / 2048 plans are for: the plan's own, those its row groups replaced, or
+// none (nullptr).
+const pf_plan_info *tile_info(const pf_plan *p)
+{
+    if (uses_row_map(p->info.variant, p->info.tile)) return &p->info;
+    return p->tiles.tile > 0 ? &p->tiles : nullptr;
+}
+
+// Back from row groups to the tiles they replaced, with a workspace of their own.  Synchronises the default stream.
+int plan_to_tiles(pf_plan *p)
+{
+    if (tile_info(p) != &p->tiles) return PF_OK;
+    const pf_plan_info groups = p->info;
+    p->info = p->tiles;
+    p->split_ready = false;
+    const int st = plan_add_split(p);
+    if (st != PF_OK) {
+        p->info = groups;
+        p->split_ready = true;
+        return st;
+    }
+    p->n_long_rows = 0;
+    p->tiles.tile = 0;
     return PF_OK;
 }
 
@@ -1194,6 +1221,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
         if (st2 != PF_OK) return st2;
         beside = near >= 0.5;
     }
+    const pf_plan_info chosen = info;  // before row groups take its place
     if (beside) {
         const int st2 = finish_info(s, dtype, PF_FLAT, PFK_VECTOR_LONG_LANES, &info);
         if (st2 != PF_OK) return st2;
@@ -1216,6 +1244,7 @@ int plan_build(const pf_row_stats &s, const int *d_row_ptr, int m, int n, int nn
     p->n = n;
     p->nnz = nnz;
     p->info = info;
+    if (info.tile != chosen.tile && uses_row_map(chosen.variant, chosen.tile)) p->tiles = chosen;
     p->stats = s;
     // A hybrid candidate starts with no workspace: a hybrid plan keeps its error flag with its own tables and
     // runs without the split-row arrays (C5: 7 MB, 0.3 ms to allocate), which come later if
@@ -1539,10 +1568,11 @@ int pf_plan_set_keep_cached(pf_plan *plan, int keep_cached)
 int pf_plan_set_row_aligned(pf_plan *plan, int row_aligned)
 {
     if (!plan || (row_aligned != 0 && row_aligned != 1)) return fail(PF_ERR_INVALID, "row_aligned must be 0 or 1");
-    if (!uses_row_map(plan->info.variant, plan->info.tile))
-        return fail(PF_ERR_UNSUPPORTED, "row-aligned tiles are FLAT 1024 or 2048");
+    if (!tile_info(plan)) return fail(PF_ERR_UNSUPPORTED, "row-aligned tiles are FLAT 1024 or 2048");
     if (row_aligned && plan->stats.max_row_len > PFK_ALIGN_ROW_MAX)
         return fail(PF_ERR_INVALID, "a row holds more than " + std::to_string(PFK_ALIGN_ROW_MAX) + " nnz");
+    const int st = plan_to_tiles(plan);
+    if (st != PF_OK) return st;
     plan->info.row_aligned = row_aligned;
     plan->info.needs_fixup = row_aligned ? 0 : (plan->info.ntiles > 1);
     if (row_aligned) plan->info.x_windows = 0;
@@ -1553,8 +1583,11 @@ int pf_plan_set_row_aligned(pf_plan *plan, int row_aligned)
 int pf_plan_set_x_windows(pf_plan *plan, int x_windows)
 {
     if (!plan || (x_windows != 0 && x_windows != 1)) return fail(PF_ERR_INVALID, "x_windows must be 0 or 1");
-    if (!uses_row_map(plan->info.variant, plan->info.tile) || (x_windows && plan->info.row_aligned))
+    const pf_plan_info *tiles = tile_info(plan);
+    if (!tiles || (x_windows && tiles->row_aligned))
         return fail(PF_ERR_UNSUPPORTED, "x-window schedules are for split-row FLAT 1024 or 2048 plans");
+    const int st = plan_to_tiles(plan);
+    if (st != PF_OK) return st;
     if (x_windows && !plan->info.x_windows) plan->map_ready = false;  // the next call records the schedule
     plan->info.x_windows = x_windows;
     return PF_OK;
@@ -1563,8 +1596,9 @@ int pf_plan_set_x_windows(pf_plan *plan, int x_windows)
 int pf_plan_set_chunk_nnz(pf_plan *plan, long long chunk_nnz)
 {
     if (!plan || chunk_nnz < 0) return fail(PF_ERR_INVALID, "chunk_nnz must be 0 or positive");
-    if (!uses_row_map(plan->info.variant, plan->info.tile))
-        return fail(PF_ERR_UNSUPPORTED, "XCD chunks are for FLAT 1024 or 2048 plans");
+    if (!tile_info(plan)) return fail(PF_ERR_UNSUPPORTED, "XCD chunks are for FLAT 1024 or 2048 plans");
+    const int st = plan_to_tiles(plan);
+    if (st != PF_OK) return st;
     plan->info.chunk_nnz = chunk_nnz;
     set_grid(plan->info);
     return PF_OK;

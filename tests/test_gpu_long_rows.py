@@ -115,6 +115,57 @@ def test_autotune_tells_the_plan_from_plain_row_groups():
         assert np.array_equal(y.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("kind", ["beside", "scattered"])
+@pytest.mark.parametrize("what", ["chunk", "row_aligned", "x_windows"])
+def test_tile_settings_take_row_groups_back_to_tiles(kind, what):
+    """The settings of FLAT tiles on a plan whose tiles gave way to row groups: the tiles', with their y bit for bit;
+    a refused value leaves the plan as it is."""
+    if kind == "beside":
+        rp, col, n = _matrix("adjacent")
+    else:
+        n, rng = 270001, np.random.default_rng(4)
+        rp = (np.arange(n + 1) * 12).astype(np.int32)
+        col = np.sort(rng.integers(0, n, (n, 12)), axis=1).astype(np.int32).ravel()
+    m, nnz, rng = len(rp) - 1, len(col), np.random.default_rng(5)
+    d = [dev(a) for a in (rp, col, rng.uniform(-1, 1, nnz), rng.uniform(-1, 1, n))]
+    ys = [torch.full((m,), float("nan"), dtype=torch.float64, device=DEV) for _ in range(2)]
+    with pf.Plan(d[0], d[1], m, n, nnz) as p:
+        assert p.info.tile == 16
+        p.execute(*d, ys[0])
+        refused = [lambda: p.set_chunk_nnz(-1), lambda: p.set_row_aligned(True) if kind == "beside" else p.set_x_windows(True)]
+        for f in refused:
+            with pytest.raises(pf.PrefreeError):
+                f()
+        assert p.info.tile == 16
+        {"chunk": lambda: p.set_chunk_nnz(8192), "row_aligned": lambda: p.set_row_aligned(False),
+         "x_windows": lambda: p.set_x_windows(kind == "beside")}[what]()
+        info = p.info
+        assert info.tile in (1024, 2048) and info.dense_rows == 0
+        assert info.chunk_nnz == 8192 if what == "chunk" else True
+        with pf.Plan(d[0], d[1], m, n, nnz, "f64", "flat", info.tile) as q:
+            q.set_chunk_nnz(info.chunk_nnz)
+            q.set_row_aligned(info.row_aligned)
+            q.set_x_windows(info.x_windows)
+            for _ in range(2):  # searched, then read from the map
+                for plan, y in ((p, ys[0]), (q, ys[1])):
+                    y.fill_(float("nan"))
+                    plan.execute(*d, y)
+                assert torch.equal(ys[0], ys[1])
+                p.check()
+        assert_parity(rp, col, d[2].cpu().numpy(), d[3].cpu().numpy(), ys[0].cpu().numpy(), "f64", what=f"{kind} {what}")
+
+
+def test_tile_settings_stay_refused_on_small_row_groups():
+    rp, col, v = pf.synth_csr(1, seed=2)
+    d = [dev(rp), dev(col)]
+    with pf.Plan(d[0], d[1], 4096, 4096, len(col)) as p:
+        assert p.info.tile == 16
+        for f in (lambda: p.set_chunk_nnz(8192), lambda: p.set_row_aligned(False), lambda: p.set_x_windows(False)):
+            with pytest.raises(pf.PrefreeError) as e:
+                f()
+            assert pf.STATUS[e.value.status] == "PF_ERR_UNSUPPORTED"
+
+
 def _stencil_with_long_rows(points, side, nlong, length, seed=3):
     """`points` columns a row around it on a side x side x side (27) or side x side grid (16), random ones (0: 27
     a row; -w: 24 a row within w of it, of `side` rows), and nlong rows of `length` random columns among them."""
