@@ -70,6 +70,23 @@ def test_hybrid_shapes(name, dtype):
     assert_parity(rp, col, val, x, y, dtype, what=f"{name}/random")
 
 
+@pytest.mark.parametrize("dtype,n,least,hybrid", [
+    ("f64", 200000, 6249, 0), ("f64", 200000, 6250, 1), ("f64", 200000, 8191, 1),   # 256 n / 8192 = 6250
+    ("f64", 131072, 4095, 0), ("f64", 131072, 4096, 1),                             # 4096 at least
+    ("f32", 400000, 6249, 0), ("f32", 400000, 6250, 1)])                            # 256 n / 16384
+def test_dense_row_threshold(dtype, n, least, hybrid):
+    """The shortest dense row at the threshold, between powers of two; x within one XCD's L2, so that a matrix below
+    it stays split-row."""
+    rng = np.random.default_rng(12)
+    lengths = [int(v) for v in rng.integers(0, 20, 900)]
+    lengths[100], lengths[101], lengths[700] = least, 9000, 12000
+    rp, col = csr_from_lengths(lengths, n, rng)
+    val, x = oracle.initvec(len(col), NP[dtype]), oracle.initvec(n, NP[dtype])
+    y, info = gpu_spmv(rp, col, val, x, "flat", dtype=dtype)
+    assert (info["hybrid"], info["dense_rows"], info["long_tiles"]) == (hybrid, 3 * hybrid, 0), info
+    assert_parity(rp, col, val, x, y, dtype, exact=kat_exact_possible(rp, dtype), what=f"{dtype} {n} {least}")
+
+
 @pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
 def test_hybrid_scaled_c5(dtype):
     rp, col, v = pf.synth_csr(5, seed=9, scale_n=200000, dtypes=(dtype,))

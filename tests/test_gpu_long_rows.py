@@ -8,7 +8,7 @@ import torch
 import oracle
 import prefree_amd as pf
 from csr_cases import csr_from_lengths
-from gpu_util import DEV, NP, TORCH, assert_parity, dev, gpu_spmv, kat_exact_possible
+from gpu_util import DEV, NP, assert_parity, dev, gpu_spmv, kat_exact_possible
 
 pytestmark = pytest.mark.gpu
 

@@ -1,10 +1,12 @@
-"""pf_spmv_noalloc (the entry point that allocates nothing) against pf_spmv, through the C ABI.
+"""pf_spmv_noalloc (the entry point that allocates nothing) against plans, pf_spmv and the oracle, through the C ABI.
 
 pf_spmv_noalloc takes its statistics block and plan workspace from the
 library's fixed device scratch array.  Two calls in a row, the second on a
-smaller matrix, must each give exactly pf_spmv's y (same plan choice, same
-kernels: bit for bit; PREFREE on known-answer values, whose sums are exact in
-any order).  The scratch keeps the previous call's contents, so the second
+smaller matrix, must each give exactly the y of a plan with a workspace of its
+own (same choice, same kernels: bit for bit; PREFREE on known-answer values,
+whose sums are exact in any order) and of pf_spmv, within the oracle's bounds.
+A tuning table keeps the plan to what the row statistics choose, as
+pf_spmv_noalloc and pf_spmv do: no hybrid plan, no row groups beside long rows.  The scratch keeps the previous call's contents, so the second
 call also checks that everything that must start cleared is cleared.
 """
 import ctypes
@@ -15,9 +17,18 @@ import torch
 
 import oracle
 import prefree_amd as pf
-from gpu_util import DEV, NP, TORCH, dev
+from gpu_util import DEV, NP, TORCH, assert_parity, dev, kat_exact_possible
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def statistics_alone(tmp_path):
+    t = tmp_path / "table.txt"
+    t.write_text("".join(f"t -1 {rows} {d} flat 1024 0 0 0 0\n" for rows in ("skewed", "dense") for d in ("f64", "f32")))
+    pf.set_tuning_table(str(t))
+    yield
+    pf.set_tuning_table(None)
 
 
 def _noalloc():
@@ -40,8 +51,15 @@ def _run(entry, rp, col, val, x, dtype, variant):
     return y[:m].cpu().numpy()
 
 
-def _reference(rp, col, val, x, dtype, variant):
-    return _run(lambda *a: pf.lib().pf_spmv(*a), rp, col, val, x, dtype, variant)
+def _plan(rp, col, val, x, dtype, variant):
+    """The first call of a plan with a workspace of its own."""
+    d = [dev(a) for a in (rp, col, val, x)]
+    y = torch.full((len(rp) - 1,), float("nan"), dtype=TORCH[dtype], device=DEV)
+    with pf.Plan(d[0], d[1], len(rp) - 1, len(x), len(col), dtype, variant) as p:
+        assert p.info.hybrid == 0 and p.info.dense_rows == 0
+        p.execute(*d, y)
+        p.check()
+    return y.cpu().numpy()
 
 
 # (cfg, scale) pairs: the first matrix of each pair is the larger one.
@@ -60,8 +78,10 @@ def test_noalloc_matches_pf_spmv(pair, variant, dtype):
         val = v[dtype]
         if kat:
             val, x = oracle.initvec(len(col), NP[dtype]), oracle.initvec(len(x), NP[dtype])
-        want = _reference(rp, col, val, x, dtype, variant)
-        got = _run(f, rp, col, val, x, dtype, variant)
+        got = _run(f, rp, col, val, x, dtype, variant)  # ahead of any other user of the scratch
+        want = _plan(rp, col, val, x, dtype, variant)
+        assert_parity(rp, col, val, x, got, dtype, exact=kat and kat_exact_possible(rp, dtype), what=f"C{cfg}/{variant}")
+        assert np.array_equal(_run(lambda *a: pf.lib().pf_spmv(*a), rp, col, val, x, dtype, variant), got)
         assert np.array_equal(got, want), f"C{cfg}/{variant}/{dtype}: {np.count_nonzero(got != want)} rows differ"
         if kat:
             assert np.array_equal(got, oracle.spmv_serial(rp, col, val, x))
@@ -70,7 +90,7 @@ def test_noalloc_matches_pf_spmv(pair, variant, dtype):
 
 def test_noalloc_two_host_threads():
     """Two host threads call pf_spmv_noalloc at once on their own streams and matrices, several times each:
-    the per-device lock orders their use of the one scratch array, so every result equals pf_spmv's."""
+    the per-device lock orders their use of the one scratch array, so every result equals a plan's."""
     import threading
 
     f = _noalloc()
@@ -78,7 +98,8 @@ def test_noalloc_two_host_threads():
     for cfg, scale in ((3, 200000), (5, 20000)):
         rp, col, v = pf.synth_csr(cfg, seed=7, scale_n=scale, dtypes=("f64",))
         x = pf.synth_x(cfg, len(rp) - 1, seed=7, dtypes=("f64",))["f64"]
-        want = _reference(rp, col, v["f64"], x, "f64", "auto")
+        want = _plan(rp, col, v["f64"], x, "f64", "auto")
+        assert_parity(rp, col, v["f64"], x, want, "f64", what=f"C{cfg}")
         m, n, nnz = len(rp) - 1, len(x), len(col)
         bufs = (dev(rp), dev(col), dev(v["f64"]), dev(x))
         y = torch.full((m,), float("nan"), dtype=torch.float64, device=DEV)
