@@ -1217,15 +1217,17 @@ struct FlatShape {
     static_assert(kVPT * 4 * kBS == K, "K must be a multiple of 1024");
 };
 
-template <typename T, int K, int MODE, bool EARLY_RP = false>
+// SHORT_ROWS (kFlatMemo): under 16 nnz per row on average, many rows per tile.  Decides two things, both measured on
+// matrices on either side: when row_ptr is loaded, and fp16's element layout.
+template <typename T, int K, int MODE, bool SHORT_ROWS = false>
 __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, int *__restrict__ dbg)
 {
     using S = FlatShape<T, K>;
     constexpr int VPT = S::kVPT;
     constexpr bool DESC = MODE == kFlatDesc;
-    // fp16 too where rows are long (not EARLY_RP): a gather over 64 consecutive nnz touches fewer x lines there
+    // fp16 too where rows are long (not SHORT_ROWS): a gather over 64 consecutive nnz touches fewer x lines there
     // (300,000 rows, 300 dense, fp16: 93.5 -> 83.1 us; short power-law rows lose, 42.9 -> 43.8).
-    constexpr bool kStrided = strided_layout<T>() || (MODE == kFlatMemo && !EARLY_RP);
+    constexpr bool kStrided = strided_layout<T>() || (MODE == kFlatMemo && !SHORT_ROWS);
     using P = acc_t<T>;
     __shared__ __attribute__((aligned(16))) P s_prod[DESC ? 4 : K + kSumPad];
     __shared__ int s_rp[DESC ? 4 : S::kRpCap];
@@ -1245,7 +1247,7 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
     const uint32_t ke = last ? (uint32_t)nnz + 1u : (uint32_t)(kb + K);
 
     // kFlatMemo: every wave reads the recorded rows itself (a uniform load), so its row_ptr loads need no barrier:
-    // ahead of the gathers (EARLY_RP) where rows are short and many, right behind them elsewhere, where waiting for
+    // ahead of the gathers (SHORT_ROWS) where rows are short and many, right behind them elsewhere, where waiting for
     // the map first would hold the gathers back (300,000 rows, 300 dense, fp64: 138 us early, 133 late; power law,
     // 400,001 rows, fp32: 24.1 early, 24.9 late).  One lane reading the map, and row_ptr after a barrier, took 137
     // and 26.5 us.
@@ -1298,7 +1300,7 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
                 load4(rc, rv, tid + k * kBS, c[k], v[k]);
             }
         }
-        if constexpr (MODE == kFlatMemo && EARLY_RP) rp_loads();
+        if constexpr (MODE == kFlatMemo && SHORT_ROWS) rp_loads();
         // The x gathers depend on col only: in the search mode they are issued
         // before the rows are known and stay in flight across the row search
         // and its barrier, which fences LDS only.  Slots past the tile read
@@ -1310,7 +1312,7 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
             for (int j = 0; j < 4; ++j)
                 xv[k][j] = buf_load(rx, tile_elem<T, kStrided>(k, j) < B - kb ? (uint32_t)c[k][j] * (uint32_t)sizeof(T) : kOob,
                                     (T *)nullptr);
-        if constexpr (MODE == kFlatMemo && !EARLY_RP) rp_loads();
+        if constexpr (MODE == kFlatMemo && !SHORT_ROWS) rp_loads();
     }
     if (MODE == kFlatMemo) {
         // nothing to search
@@ -1388,7 +1390,8 @@ __global__ __launch_bounds__(kBS) void k_flat(Args<T> a, int *__restrict__ map, 
             else if (tail && i == nr - 1) a.tail[t] = s;
             else a.y[lo_row + i] = T(s);
         });
-    if (tid == 0) a.owner[t] = tail ? lo_row + nr - 1 : -1;
+    // k_fixup's owner slot; with a recorded map k_fixup_map takes the split rows from the map
+    if (MODE != kFlatMemo && tid == 0) a.owner[t] = tail ? lo_row + nr - 1 : -1;
 }
 
 // ---- k_rows: FLAT tiles that own whole rows --------------------------------
