@@ -4,8 +4,8 @@
 One step = one y = A·x (pf_plan_execute) over the whole matrix, inputs already
 resident in HBM.  The headline (`value`, `roofline`, `cpu_baseline`) is C5, the
 largest single-GPU configuration of BASELINE.json (mixed dense rows, n = 10^6,
-about 316M nnz, fp64); `configs` holds the same record for C1, C2, C3, C4,
-C4 in fp32 and C5.  --config N measures configuration N alone (and makes it
+about 316M nnz, fp64); `configs` holds the main figures of C1, C2, C3, C4,
+C4 in fp32 and C5, and --records FILE writes every configuration's whole record.  --config N measures configuration N alone (and makes it
 the headline).
 
 Per configuration:
@@ -29,7 +29,7 @@ Per configuration:
 `kernel_ms`; `roofline.traffic` the HBM bytes per step measured by rocprofv3
 (profiles/traffic.json) when committed for that plan.
 
-Prints ONE JSON line.
+Prints ONE JSON line, of about four thousand characters.
 """
 from __future__ import annotations
 
@@ -563,6 +563,8 @@ def main():
                     help="gather: time the x gathers alone (random indices and each configuration's columns) "
                          "instead of the SpMV")
     ap.add_argument("--probe-reps", type=int, default=50)
+    ap.add_argument("--records", default="", metavar="FILE",
+                    help="write the whole record of every configuration to FILE (JSON)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="after the measurement, run a plain copy kernel over 256 MiB 3 times (known bytes, "
                          "for scaling rocprofv3 FETCH_SIZE / WRITE_SIZE readings)")
@@ -607,7 +609,10 @@ def main():
         torch.cuda.synchronize()
         del src, dst
 
-    h = records[cfg_name(*head)]
+    if args.records:
+        with open(args.records, "w") as f:
+            json.dump(records, f, indent=1)
+    h = without_text(records[cfg_name(*head)])
     result = {
         "metric": METRIC,
         "value": h["gflops"],
@@ -642,15 +647,36 @@ def main():
         "cpu_baseline": h["cpu_baseline"],
         "parity": h.get("parity"),
         "speedup_vs_cpu": h.get("speedup_vs_cpu"),
-        "configs": records,
+        "configs": {name: main_figures(r) for name, r in records.items()},
     }
     print(json.dumps(result), flush=True)
     print_summary(records)
 
 
+def without_text(rec):
+    """A record without the sentences that explain its fields (the module docstring has them)."""
+    return {k: {a: b for a, b in v.items() if a not in ("what", "note")} if isinstance(v, dict) else v
+            for k, v in rec.items()}
+
+
+def main_figures(r):
+    """A configuration's figures for the JSON line."""
+    def part(name, key):
+        return (r.get(name) or {}).get(key)
+
+    return {"plan": plan_name(r), "ms": r["ms"], "kernel_ms": r["kernel_ms"], "gflops": r["gflops"],
+            "frac": r["roofline"]["frac"], "rotated_ms": part("rotated", "kernel_ms"), "cold_ms": part("cold", "ms"),
+            "search_x": part("search", "vs_recorded_rows"), "plan_ms": r["plan_ms"], "parity_ok": part("parity", "ok")}
+
+
+def plan_name(r):
+    return r["variant"] + f"-{r['tile']}" + ("-rows" if r["row_aligned"] else "") + (
+        f"-band{r['band_w']}" if r.get("band_w") else "") + (
+        ("-long" if r["long_tiles"] else "-dense") + ("-halves" if r["x_halves"] else "") if r["hybrid"] else "")
+
+
 def print_summary(records):
-    """One short line per configuration on stderr, after the JSON line: a reader of the end of the output
-    sees every configuration even when the start of the long JSON line is cut off."""
+    """One short line per configuration on stderr, after the JSON line."""
     def f(v, fmt):
         return format(v, fmt) if isinstance(v, (int, float)) else "-"
 
@@ -658,10 +684,7 @@ def print_summary(records):
         rot, cold, srch = r.get("rotated") or {}, r.get("cold") or {}, r.get("search") or {}
         roof, par, cpu = r["roofline"], r.get("parity") or {}, r.get("cpu_baseline") or {}
         ratio = roof["traffic"] / roof["algorithmic_bytes"] if roof.get("traffic") else None
-        plan = r["variant"] + f"-{r['tile']}" + ("-rows" if r["row_aligned"] else "") + (
-            f"-band{r['band_w']}" if r.get("band_w") else "") + (
-            ("-long" if r["long_tiles"] else "-dense") + ("-halves" if r["x_halves"] else "") if r["hybrid"] else "")
-        print(f"summary {name}: plan={plan} kernel_us={f(r['kernel_ms'] * 1e3, '.2f')} "
+        print(f"summary {name}: plan={plan_name(r)} kernel_us={f(r['kernel_ms'] * 1e3, '.2f')} "
               f"frac={f(roof['frac'], '.4f')} rotated_frac={f(rot.get('frac'), '.4f')} "
               f"cold_frac={f(cold.get('frac'), '.4f')} search_x={f(srch.get('vs_recorded_rows'), '.3f')} "
               f"traffic_ratio={f(ratio, '.2f')} plan_ms={f(r['plan_ms'], '.3f')} "
