@@ -3382,7 +3382,8 @@ __global__ __launch_bounds__(kBS) void k_row_map(const int *__restrict__ rp, int
 // swizzle tree adds the L lane sums, and the group's first lane stores y.
 // Every index is clamped to the matrix: a row_ptr changed after planning reads
 // in bounds.  C1 in a HIP graph: 1.85 us per SpMV with L = 16 against 3.50 for
-// 1024-nnz tiles (2.49 in a launch loop against 2.73 for rocSPARSE's row split).
+// 1024-nnz tiles; a launch loop is bound by the host (3.1-3.8 us per call, 2.49 on one box against 2.73 for
+// rocSPARSE's row split).
 template <typename T, int L>
 __global__ __launch_bounds__(kBS) void k_vector(Args<T> a)
 {

@@ -1955,8 +1955,8 @@ const char *pf_tuning_table(void)
 }
 
 // An eager call under kGraphTimeUs is bound by the host's launch rate, which hides the kernels' differences
-// (C1: about 3.9 us per call for every candidate launched one by one; in a graph, 1.96 us for 16-lane row groups
-// and 3.60 for 1024-nnz tiles).  pf_plan_autotune then times every candidate as a captured graph.
+// (C1: 3.1-3.9 us per call from box to box, whatever the candidate, launched one by one; in a graph, 1.96 us for
+// 16-lane row groups and 3.60 for 1024-nnz tiles).  pf_plan_autotune then times every candidate as a captured graph.
 constexpr double kGraphTimeUs = 20.0;
 
 // Mean us per call of `reps` back-to-back calls on `stream`, the best of two batches, each batch launched
